@@ -1089,7 +1089,7 @@ extern "C" void *gz_gpu_build_scene(const PrimId_C *prims, int64_t nPrims, const
                   dalloc(&keys2, n, "build keys") && dalloc(&vals, n, "build order") && dalloc(&vals2, n, "build order") &&
                   dalloc(&node, m, "build nodes") && dalloc(&rec, m, "build subtree records") &&
                   dalloc(&sortedPrims, n, "build primIds") &&
-                  dalloc(&s->dTris, n, "build triangle records") && dalloc(&s->dNodes, m, "build node records") &&
+                  dalloc(&s->dTris, (size_t)n + 1, "build triangle records") && dalloc(&s->dNodes, m, "build node records") &&
                   (!sah || (dalloc(&bigA, n, "build SAH tasks") && dalloc(&bigB, n, "build SAH tasks") &&
                             dalloc(&smallTasks, n, "build SAH tasks") && dalloc(&sahCounters, 4, "build SAH counters") &&
                             dalloc(&leafMark, m, "build SAH leaves")));

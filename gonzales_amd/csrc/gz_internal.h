@@ -31,6 +31,8 @@ static_assert(sizeof(NodePair) == 64, "NodePair");
 //   p1.w : index into primIds of this primitive (the reference's hitIndex), as int bits
 //   p2.w : flags as int bits; bit 0 = skip (the reference `continue`s: id2 == -1 or an
 //          unknown type, kernel.mojo:273-277)
+// The array holds one record more than there are primitives: a traversal step loads 64 bytes at a
+// record, so at the last one 16 bytes past it.
 struct alignas(16) TriRec {
         float4 p0;
         float4 p1;

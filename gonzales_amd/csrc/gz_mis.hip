@@ -501,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_wf_rays(MisArgs a, const GzPath *__r
                         int st;
                         do {
                                 st = step<kAny, kStats, kLdsMax>(L, S, a.nodes, a.tris);
-                        } while (st == kStepGo && !(kMode == 2 && L.hitPrim >= 0 && L.tBest < tStop));
+                        } while (st == kStepGo && !(kMode == 2 && L.hitPrim >= 0 && L.left == 0 && L.tBest < tStop));
                         if (st == kStepOverflow) {
                                 atomicOr(a.err, 1);
                                 L.hitPrim = -1;

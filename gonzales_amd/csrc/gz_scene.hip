@@ -306,7 +306,7 @@ extern "C" void *gz_gpu_upload_scene(const BVH2Node *nodes, int64_t nNodes, cons
                                 p.d = make_int4(recOf[(size_t)(i + 1)], recOf[(size_t)nodes[i].offset], 0, 0);
                         }
                         // Triangle records, leaf by leaf.
-                        tris.resize((size_t)triNext);
+                        tris.resize((size_t)triNext + 1);  // one more: step() loads 64 bytes at a record
                         for (int64_t i = 0; i < nNodes; ++i) {
                                 const int32_t rec = recOf[(size_t)i];
                                 if (rec == INT32_MIN || rec >= 0) continue;

@@ -148,7 +148,7 @@ __device__ __forceinline__ bool trace_ray_until(const MisArgs &a, const Ray_C &r
         int st;
         do {
                 st = step<false, kStats, kLdsMis>(L, w.S, a.nodes, a.tris);
-        } while (st == kStepGo && !(L.hitPrim >= 0 && L.tBest < tStop));
+        } while (st == kStepGo && !(L.hitPrim >= 0 && L.left == 0 && L.tBest < tStop));
         if (kStats) {
                 w.interior += L.nInterior;
                 w.tris += L.nTris;
