@@ -351,10 +351,10 @@ __global__ __launch_bounds__(kMisBlock) void k_bw_rays(const int *__restrict__ c
                         if (kMode == 0) {
                                 const GzPath &p = paths[idx];
                                 trace = path_live(a, p);
-                                if (trace) lane_init(L, p.ray, INFINITY, a.rootDesc, a.sceneSafe);
+                                if (trace) lane_init(L, p.ray, INFINITY, a.rootDesc, a.boxes);
                         } else {
                                 lane_init(L, kAny ? ws.srays[idx] : ws.mrays[idx], kAny ? 1.0f - 0.00001f : INFINITY,
-                                          a.rootDesc, a.sceneSafe);
+                                          a.rootDesc, a.boxes);
                         }
                         if (trace && !a.empty) {
                                 int st;

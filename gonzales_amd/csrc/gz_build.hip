@@ -1208,7 +1208,8 @@ extern "C" void *gz_gpu_build_scene(const PrimId_C *prims, int64_t nPrims, const
                 const bool rootLeaf = sah ? h[1] == 0 : n <= maxLeaf;
                 s->nodeRecords = rootLeaf ? 0 : h[1];  // records numbered depth first, densely
                 s->triCount = n;
-                s->boundsSafe = !(h[0] & (kFlagUnsafe | kFlagSkip));  // finite boxes within 2^40, none empty
+                // finite boxes within 2^40, none empty; min/max of what they hold, so nested
+                s->boxes = (h[0] & (kFlagUnsafe | kFlagSkip)) ? 0 : kBoxesBounded | kBoxesNested;
                 if (rootLeaf) {
                         s->rootDesc = ~0;
                         s->interiorCount = 0;

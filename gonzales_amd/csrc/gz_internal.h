@@ -42,6 +42,10 @@ static_assert(sizeof(TriRec) == 48, "TriRec");
 
 enum : int { kTriSkip = 1 };
 
+// Scene::boxes. Bounded: every box coordinate is finite with magnitude <= 2^40. Nested: every box that
+// a traversal tests holds its children's boxes or, for a leaf, the vertices of its triangles.
+enum : int { kBoxesBounded = 1, kBoxesNested = 2 };
+
 // Device-resident mesh view for the shading kernels: TriangleMesh_C's pointers plus the element
 // counts passed at upload, so a kernel can reject an index the reference would read past.
 struct DevMesh {
@@ -125,7 +129,7 @@ struct Scene {
 
         // Traversal launch configuration.
         GzTraceConfig traceConfig{3, 16, 32, 1, 128, 1 << 18, 0, 0};
-        bool boundsSafe = false;  // every node box coordinate is finite with magnitude <= 2^40
+        int boxes = 0;  // what is known of the node boxes: kBoxesBounded | kBoxesNested
         int cuCount = 256;
 };
 

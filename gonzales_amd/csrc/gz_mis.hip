@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kBlock) void k_wf_trace(MisArgs a, const GzPath *__
                                                 cur = qin ? qin[mine] : (int)mine;
                                                 const GzPath &p = paths[cur];
                                                 if (path_live(a, p)) {
-                                                        lane_init(L, p.ray, INFINITY, a.rootDesc, a.sceneSafe);
+                                                        lane_init(L, p.ray, INFINITY, a.rootDesc, a.boxes);
                                                         done = a.empty;  // no nodes: a miss, nothing to step
                                                 } else {
                                                         L.hitPrim = -1;
@@ -491,9 +491,9 @@ __global__ __launch_bounds__(kBlock) void k_wf_rays(MisArgs a, const GzPath *__r
                 if (kMode == 0) {
                         const GzPath &p = paths[idx];
                         trace = path_live(a, p);
-                        if (trace) lane_init(L, p.ray, INFINITY, a.rootDesc, a.sceneSafe);
+                        if (trace) lane_init(L, p.ray, INFINITY, a.rootDesc, a.boxes);
                 } else {
-                        lane_init(L, rays[idx], kAny ? 1.0f - 0.00001f : INFINITY, a.rootDesc, a.sceneSafe);
+                        lane_init(L, rays[idx], kAny ? 1.0f - 0.00001f : INFINITY, a.rootDesc, a.boxes);
                 }
                 if (trace && !a.empty) {
                         // BSDF rays stop at a hit closer than the emitter box (bsdf_ray_stop)
@@ -1033,7 +1033,7 @@ bool gz::mis_args(Scene *s, const GzMisParams *params, int *err, MisArgs &a) {
         a.nodes = s->dNodes;
         a.tris = s->dTris;
         a.rootDesc = s->rootDesc;
-        a.sceneSafe = s->boundsSafe;
+        a.boxes = s->boxes;
         a.empty = s->empty;
         a.prims = s->dPrims;
         a.primCount = s->primCount;

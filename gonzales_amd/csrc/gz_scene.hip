@@ -81,6 +81,8 @@ int check_stream(Scene *s, hipStream_t st) {
         return GZ_E_INVALID;
 }
 
+constexpr int kUploadBlock = 256;
+
 static void free_scene(Scene *s) {
         if (!s) return;
         int cur = -1;
@@ -162,6 +164,58 @@ bool scene_upload_common(Scene *s, const PrimId_C *prims, int64_t nPrims, const 
 }
 
 void scene_release(Scene *s) { free_scene(s); }
+
+// Raises bit 2 of *flag if a box tested at record k does not hold what is under it: the boxes of an
+// interior child's children, the vertices of a leaf child's triangles. (The root's own box is never
+// tested.) The boxes come from the caller, so this is looked at and not assumed; on the device because
+// the host walk took 37 ms of a million-triangle upload.
+__global__ __launch_bounds__(kUploadBlock) void k_nested(const NodePair *__restrict__ nodes, int64_t n,
+                                                         const TriRec *__restrict__ tris, int *__restrict__ flag) {
+        const int64_t k = (int64_t)blockIdx.x * kUploadBlock + threadIdx.x;
+        if (k >= n) return;
+        const NodePair p = nodes[k];
+        const float lo[2][3] = {{p.a.x, p.a.y, p.a.z}, {p.b.z, p.b.w, p.c.x}};
+        const float hi[2][3] = {{p.a.w, p.b.x, p.b.y}, {p.c.y, p.c.z, p.c.w}};
+        bool ok = true;
+        for (int side = 0; side < 2; ++side) {
+                auto holds = [&](float x, float y, float z) {
+                        return x >= lo[side][0] && x <= hi[side][0] && y >= lo[side][1] && y <= hi[side][1] &&
+                               z >= lo[side][2] && z <= hi[side][2];
+                };
+                const int c = side ? p.d.y : p.d.x;
+                if (c >= 0) {
+                        const NodePair q = nodes[c];
+                        ok = ok && holds(q.a.x, q.a.y, q.a.z) && holds(q.a.w, q.b.x, q.b.y) && holds(q.b.z, q.b.w, q.c.x) &&
+                             holds(q.c.y, q.c.z, q.c.w);
+                        continue;
+                }
+                const TriRec *leaf = tris + ~c;
+                const int count = __float_as_int(leaf[0].p0.w);
+                for (int j = 0; ok && j < count; ++j) {
+                        const TriRec t = leaf[j];
+                        if (__float_as_int(t.p2.w) & kTriSkip) continue;
+                        ok = holds(t.p0.x, t.p0.y, t.p0.z) && holds(t.p1.x, t.p1.y, t.p1.z) && holds(t.p2.x, t.p2.y, t.p2.z);
+                }
+        }
+        if (!ok) atomicOr(flag, 4);
+}
+
+// Sets kBoxesNested of an uploaded scene (its stream's error word carries the answer).
+static bool find_nested(Scene *s) {
+        if (s->nodeRecords <= 0) return true;
+        StreamSlot *slot = stream_slot(s, s->stream);
+        if (!slot) return false;
+        int flag = 0;
+        hipLaunchKernelGGL(k_nested, dim3((unsigned)((s->nodeRecords + kUploadBlock - 1) / kUploadBlock)),
+                           dim3(kUploadBlock), 0, s->stream, s->dNodes, s->nodeRecords, s->dTris, slot->dErr);
+        if (!hip_ok(hipGetLastError(), "box check") ||
+            !hip_ok(hipMemcpyAsync(&flag, slot->dErr, sizeof flag, hipMemcpyDeviceToHost, s->stream), "box check") ||
+            !hip_ok(hipMemsetAsync(slot->dErr, 0, sizeof flag, s->stream), "box check") ||
+            !hip_ok(hipStreamSynchronize(s->stream), "box check"))
+                return false;
+        if (!(flag & 4)) s->boxes |= kBoxesNested;
+        return true;
+}
 
 static inline int32_t as_int(float f) {
         int32_t i;
@@ -291,7 +345,6 @@ extern "C" void *gz_gpu_upload_scene(const BVH2Node *nodes, int64_t nNodes, cons
                                                 if (!(x >= -0x1p40f && x <= 0x1p40f)) safe = false;
                                 }
                         }
-                        s->boundsSafe = safe;
                         s->triCount = triNext;
                         s->rootDesc = recOf[0];
                         pairs.resize(order.size());
@@ -360,6 +413,7 @@ extern "C" void *gz_gpu_upload_scene(const BVH2Node *nodes, int64_t nNodes, cons
                                         t.p2.w = as_float(flags);
                                 }
                         }
+                        s->boxes = safe ? kBoxesBounded : 0;
                 }
         } catch (const std::bad_alloc &) {
                 if (gz_last_error()[0] == 0) set_error("gz_gpu_upload_scene: out of host memory");
@@ -372,7 +426,8 @@ extern "C" void *gz_gpu_upload_scene(const BVH2Node *nodes, int64_t nNodes, cons
                   upload(&s->dNodes, pairs.data(), (int64_t)pairs.size(), s, "upload nodes") &&
                   upload(&s->dTris, tris.data(), (int64_t)tris.size(), s, "upload triangles") &&
                   scene_upload_common(s, prims, nPrims, meshes, nMeshes, ptsCounts, faceCounts, vtxCounts, materials,
-                                      nMaterials);
+                                      nMaterials) &&
+                  find_nested(s);
         if (!ok) {
                 free_scene(s);
                 return nullptr;

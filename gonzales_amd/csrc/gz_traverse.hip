@@ -33,17 +33,17 @@ struct alignas(16) SortedRay {
 
 // Starts lane L on entry j of a binned batch; returns the ray's index in the caller's arrays.
 __device__ __forceinline__ int64_t lane_start_sorted(Lane &L, const SortedRay *__restrict__ sorted, int64_t j,
-                                                     int rootDesc, bool sceneSafe) {
+                                                     int rootDesc, int boxes) {
         const SortedRay r = sorted[j];
         const Ray_C ray{r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y};
-        lane_init(L, ray, r.b.z, rootDesc, sceneSafe);
+        lane_init(L, ray, r.b.z, rootDesc, boxes);
         return (int64_t)__float_as_uint(r.b.w);
 }
 
 // One lane per ray, one ray per lane.
 template <bool kAny, bool kStats, int kLds>
 __global__ __launch_bounds__(kBlock) void k_trace(const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris,
-                                                  int rootDesc, bool sceneSafe, const Ray_C *__restrict__ rays,
+                                                  int rootDesc, int boxes, const Ray_C *__restrict__ rays,
                                                   const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
                                                   uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats,
                                                   int *__restrict__ err, const SortedRay *__restrict__ order) {
@@ -52,13 +52,13 @@ __global__ __launch_bounds__(kBlock) void k_trace(const NodePair *__restrict__ n
         Lane L;
         int64_t i = j;
         if (order)
-                i = lane_start_sorted(L, order, j, rootDesc, sceneSafe);
+                i = lane_start_sorted(L, order, j, rootDesc, boxes);
         else
-                lane_start(L, rays, tMaxIn, i, rootDesc, sceneSafe);
+                lane_start(L, rays, tMaxIn, i, rootDesc, boxes);
         Stack<kLds> S;
         int st;
         do {
-                st = step<kAny, kStats, kLds>(L, S, nodes, tris);
+                st = step<kAny, kStats, kLds>(L, S, nodes, tris, boxes);
         } while (st == kStepGo);
         lane_finish<kAny, kStats>(L, i, st == kStepOverflow, hits, occ, stats, err);
 }
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(const NodePair *__restrict__ n
 // other lanes of a wave. A wave leaves once the counter is exhausted and its lanes are idle.
 template <bool kAny, bool kStats, int kLds>
 __global__ __launch_bounds__(kBlock) void k_trace_persistent(
-        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, bool sceneSafe,
+        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, int boxes,
         const Ray_C *__restrict__ rays, const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
         uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats, int *__restrict__ err,
         unsigned long long *__restrict__ counter, int refill, int chunk, const SortedRay *__restrict__ order) {
@@ -112,10 +112,10 @@ __global__ __launch_bounds__(kBlock) void k_trace_persistent(
                                         if (mine < un) {
                                                 if (order) {
                                                         ray = lane_start_sorted(L, order, (int64_t)mine, rootDesc,
-                                                                                sceneSafe);
+                                                                                boxes);
                                                 } else {
                                                         ray = (int64_t)mine;
-                                                        lane_start(L, rays, tMaxIn, ray, rootDesc, sceneSafe);
+                                                        lane_start(L, rays, tMaxIn, ray, rootDesc, boxes);
                                                 }
                                         }
                                 }
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_persistent(
                         }
                 }
                 if (ray >= 0) {
-                        const int st = step<kAny, kStats, kLds>(L, S, nodes, tris);
+                        const int st = step<kAny, kStats, kLds>(L, S, nodes, tris, boxes);
                         if (st != kStepGo) {
                                 lane_finish<kAny, kStats>(L, ray, st == kStepOverflow, hits, occ, stats, err);
                                 ray = -1;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_persistent(
 // k_trace_persistent; a wave leaves once all eight ranges are handed out and its lanes are idle.
 template <bool kAny, bool kStats, int kLds>
 __global__ __launch_bounds__(kBlock) void k_trace_xcd(
-        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, bool sceneSafe,
+        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, int boxes,
         const Ray_C *__restrict__ rays, const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
         uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats, int *__restrict__ err,
         unsigned long long *__restrict__ counters, int refill, int chunk, const SortedRay *__restrict__ order) {
@@ -201,10 +201,10 @@ __global__ __launch_bounds__(kBlock) void k_trace_xcd(
                                         if (mine < un) {
                                                 if (order) {
                                                         ray = lane_start_sorted(L, order, (int64_t)mine, rootDesc,
-                                                                                sceneSafe);
+                                                                                boxes);
                                                 } else {
                                                         ray = (int64_t)mine;
-                                                        lane_start(L, rays, tMaxIn, ray, rootDesc, sceneSafe);
+                                                        lane_start(L, rays, tMaxIn, ray, rootDesc, boxes);
                                                 }
                                         }
                                 }
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_xcd(
                         }
                 }
                 if (ray >= 0) {
-                        const int st = step<kAny, kStats, kLds>(L, S, nodes, tris);
+                        const int st = step<kAny, kStats, kLds>(L, S, nodes, tris, boxes);
                         if (st != kStepGo) {
                                 lane_finish<kAny, kStats>(L, ray, st == kStepOverflow, hits, occ, stats, err);
                                 ray = -1;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_xcd(
 // consecutive rays. Each lane leaves after its last ray, so every wave exits.
 template <bool kAny, bool kStats, int kLds>
 __global__ __launch_bounds__(kBlock) void k_trace_strided(
-        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, bool sceneSafe,
+        const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris, int rootDesc, int boxes,
         const Ray_C *__restrict__ rays, const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
         uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats, int *__restrict__ err,
         const SortedRay *__restrict__ order) {
@@ -246,20 +246,20 @@ __global__ __launch_bounds__(kBlock) void k_trace_strided(
         Lane L;
         int64_t ray = j;
         if (order)
-                ray = lane_start_sorted(L, order, j, rootDesc, sceneSafe);
+                ray = lane_start_sorted(L, order, j, rootDesc, boxes);
         else
-                lane_start(L, rays, tMaxIn, ray, rootDesc, sceneSafe);
+                lane_start(L, rays, tMaxIn, ray, rootDesc, boxes);
         for (;;) {
-                const int st = step<kAny, kStats, kLds>(L, S, nodes, tris);
+                const int st = step<kAny, kStats, kLds>(L, S, nodes, tris, boxes);
                 if (st != kStepGo) {
                         lane_finish<kAny, kStats>(L, ray, st == kStepOverflow, hits, occ, stats, err);
                         j += G;
                         if (j >= n) break;
                         if (order) {
-                                ray = lane_start_sorted(L, order, j, rootDesc, sceneSafe);
+                                ray = lane_start_sorted(L, order, j, rootDesc, boxes);
                         } else {
                                 ray = j;
-                                lane_start(L, rays, tMaxIn, ray, rootDesc, sceneSafe);
+                                lane_start(L, rays, tMaxIn, ray, rootDesc, boxes);
                         }
                 }
         }
@@ -495,7 +495,7 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                 const int64_t want = (int64_t)s->cuCount * perCU * (c.gridScale > 0 ? c.gridScale : 1);
                 const unsigned g = (unsigned)std::min<int64_t>(want, grid_for(n));
                 hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, stream, s->dNodes, s->dTris, s->rootDesc,
-                                   s->boundsSafe, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, order);
+                                   s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, order);
         } else if (c.persistent == 3) {
                 auto kern = k_trace_xcd<kAny, kStats, kLds>;
                 int perCU = 0;
@@ -505,7 +505,7 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                 const unsigned g = (unsigned)std::min<int64_t>(want, grid_for(n));
                 hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, stream, slot.dCounter);
                 hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, stream, s->dNodes, s->dTris, s->rootDesc,
-                                   s->boundsSafe, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, slot.dCounter,
+                                   s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, slot.dCounter,
                                    c.refillLanes > 0 && c.refillLanes <= 64 ? c.refillLanes : 16,
                                    c.chunk >= 1 && c.chunk <= 4096 ? c.chunk : 64, order);
         } else if (c.persistent == 1) {
@@ -518,12 +518,12 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                 unsigned long long *ctr = slot.dCounter;
                 hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(1), 0, stream, ctr);
                 hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, stream, s->dNodes, s->dTris, s->rootDesc,
-                                   s->boundsSafe, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, ctr,
+                                   s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, ctr,
                                    c.refillLanes > 0 && c.refillLanes <= 64 ? c.refillLanes : 16,
                                    c.chunk >= 1 && c.chunk <= 4096 ? c.chunk : 64, order);
         } else {
                 hipLaunchKernelGGL((k_trace<kAny, kStats, kLds>), dim3(grid_for(n)), dim3(kBlock), 0, stream, s->dNodes,
-                                   s->dTris, s->rootDesc, s->boundsSafe, d_rays, d_tMax, n, d_hits, d_occ, d_stats,
+                                   s->dTris, s->rootDesc, s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats,
                                    slot.dErr, order);
         }
 }

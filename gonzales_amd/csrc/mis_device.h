@@ -47,7 +47,7 @@ struct MisArgs {
         const NodePair *nodes;
         const TriRec *tris;
         int rootDesc;
-        bool sceneSafe;
+        int boxes;  // kBoxesBounded | kBoxesNested
         bool empty;
         const PrimId_C *prims;
         int64_t primCount;
@@ -93,7 +93,7 @@ __device__ __forceinline__ bool trace_ray(const MisArgs &a, const Ray_C &ray, fl
                                           float &u, float &v, Work &w) {
         if (a.empty) return false;
         Lane L;
-        lane_init(L, ray, tMax, a.rootDesc, a.sceneSafe);
+        lane_init(L, ray, tMax, a.rootDesc, a.boxes);
         int st;
         do {
                 st = step<kAny, kStats, kLdsMis>(L, w.S, a.nodes, a.tris);
@@ -144,7 +144,7 @@ __device__ __forceinline__ bool trace_ray_until(const MisArgs &a, const Ray_C &r
                                                 float &u, float &v, Work &w) {
         if (a.empty) return false;
         Lane L;
-        lane_init(L, ray, INFINITY, a.rootDesc, a.sceneSafe);
+        lane_init(L, ray, INFINITY, a.rootDesc, a.boxes);
         int st;
         do {
                 st = step<false, kStats, kLdsMis>(L, w.S, a.nodes, a.tris);

@@ -72,6 +72,38 @@ __device__ __forceinline__ bool slab(float mnx, float mny, float mnz, float mxx,
         return slab_exact(mnx, mny, mnz, mxx, mxy, mxz, r, tMax, tNearOut);
 }
 
+// True if no triangle inside the box can pass tri_test, from an axis the ray does not move along.
+//
+// slab_exact does not cull on such an axis: 0 * inf makes its plane distances NaN there (or both
+// infinite with one sign) and the reference's selects drop them. A ray with one zero direction
+// component then visits every box that its line crosses in the other two axes: about 10,000 nodes of
+// a million-triangle soup instead of 125, in one lane, and one such ray in 16M random ones (a
+// component of torch.rand is exactly 0.5 that often) held the whole batch for 4 to 6 ms.
+//
+// The bound. With exact edges e1, e2 and offset t = origin - vertex, det t = Nu e1 + Nv e2 - Nt d
+// (Cramer), so on an axis where d is 0, t = u e1 + v e2: a triangle that does not reach the origin's
+// coordinate on that axis is only accepted through tri_test's rounding. Let E bound the edges'
+// components, T those of t, D = |dx| + |dy| + |dz| and w = 2^-24. The computed det is off by at most
+// 10 w D E^2, the numerators of u and v by 10 w D E T each, and |det| >= 1e-7 on acceptance, so the
+// accepted (u, v) miss the equation by at most 30 w D E^2 T / 1e-7 = 17.9 D E^2 T, plus a few w (E + T)
+// for the quotients, the edges, the offset and u + v <= 1. Farther away than that (20 and 1e-6 for the
+// float evaluation here) the triangle is rejected. E and T of the box bound those of its triangles, and
+// D E^2 < 1/20 where the test culls and T <= 2^41 (bounded boxes, an origin within 2^40), so no
+// intermediate of tri_test overflows to an infinity or NaN, which it would accept; a direction that is
+// not finite makes M NaN or infinite, which culls nothing.
+__device__ __forceinline__ bool beyond_zero_axis(float mnx, float mny, float mnz, float mxx, float mxy, float mxz,
+                                                 const RayState &r) {
+        const float lx = mnx - r.ox, ly = mny - r.oy, lz = mnz - r.oz;
+        const float hx = r.ox - mxx, hy = r.oy - mxy, hz = r.oz - mxz;
+        const float E = fmaxf(fmaxf(mxx - mnx, mxy - mny), mxz - mnz);
+        const float T = fmaxf(fmaxf(fmaxf(fabsf(lx), fabsf(hx)), fmaxf(fabsf(ly), fabsf(hy))), fmaxf(fabsf(lz), fabsf(hz)));
+        const float D = (fabsf(r.dx) + fabsf(r.dy)) + fabsf(r.dz);
+        const float M = 20.0f * (D * (E * E)) * T + 1e-6f * (E + T);
+        if (!(fabsf(r.ox) <= 0x1p40f && fabsf(r.oy) <= 0x1p40f && fabsf(r.oz) <= 0x1p40f)) return false;
+        return (r.dx == 0.0f && (lx > M || hx > M)) || (r.dy == 0.0f && (ly > M || hy > M)) ||
+               (r.dz == 0.0f && (lz > M || hz > M));
+}
+
 // v_max3_f32 / v_min3_f32 of three values none of which is NaN. fmaxf and fminf of the same values
 // give the same results (up to the sign of a zero), but the compiler quiets each operand with an
 // extra v_max_f32 first (IEEE mode), which doubles the work of the slab test.
@@ -147,14 +179,14 @@ struct Lane {
         uint32_t nInterior, nTris;
 };
 
-__device__ __forceinline__ void lane_init(Lane &L, const Ray_C ray, float tMax, int rootDesc, bool sceneSafe);
+__device__ __forceinline__ void lane_init(Lane &L, const Ray_C ray, float tMax, int rootDesc, int boxes);
 
 __device__ __forceinline__ void lane_start(Lane &L, const Ray_C *__restrict__ rays, const float *__restrict__ tMaxIn,
-                                           int64_t i, int rootDesc, bool sceneSafe) {
-        lane_init(L, rays[i], tMaxIn[i], rootDesc, sceneSafe);
+                                           int64_t i, int rootDesc, int boxes) {
+        lane_init(L, rays[i], tMaxIn[i], rootDesc, boxes);
 }
 
-__device__ __forceinline__ void lane_init(Lane &L, const Ray_C ray, float tMax, int rootDesc, bool sceneSafe) {
+__device__ __forceinline__ void lane_init(Lane &L, const Ray_C ray, float tMax, int rootDesc, int boxes) {
         L.tMax = tMax;
         RayState &r = L.r;
         r.ox = ray.orgX;
@@ -176,7 +208,7 @@ __device__ __forceinline__ void lane_init(Lane &L, const Ray_C ray, float tMax, 
         // (checked at upload), bound every slab product and difference by 2^81: no inf, no NaN.
         const float lo = 0x1p-40f, hi = 0x1p40f;
         const float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
-        r.safe = sceneSafe && ax >= lo && ay >= lo && az >= lo && ax <= hi && ay <= hi && az <= hi &&
+        r.safe = (boxes & kBoxesBounded) && ax >= lo && ay >= lo && az >= lo && ax <= hi && ay <= hi && az <= hi &&
                  fabsf(r.ox) <= hi && fabsf(r.oy) <= hi && fabsf(r.oz) <= hi;
         L.hitPrim = -1;
         L.tBest = __builtin_canonicalizef(L.tMax);  // a signalling NaN quieted: the slab tests ignore it
@@ -198,22 +230,26 @@ constexpr int kLdsMax = 16;
 constexpr int kLdsWide = 32;
 __shared__ int g_stackLds[kLdsMax * kBlock];
 __shared__ int g_stackLdsWide[kLdsWide * kBlock];
+__shared__ int g_stackLdsWave[kLdsMax * 64];
 
 // Traversal stack of GZ_STACK_CAPACITY entries: the first kLds live in LDS, the rest in
 // per-lane private memory.
-template <int kLds>
+template <int kLds, int kWidth = kBlock>
 struct Stack {
         static_assert(kLds <= kLdsWide, "LDS stack rows");
+        static_assert(kWidth == kBlock || (kWidth == 64 && kLds <= kLdsMax), "LDS stack width");
         int priv[GZ_STACK_CAPACITY - kLds > 0 ? GZ_STACK_CAPACITY - kLds : 1];
         __device__ __forceinline__ static int *rows() {
-                if constexpr (kLds > kLdsMax)
+                if constexpr (kWidth == 64)
+                        return g_stackLdsWave;
+                else if constexpr (kLds > kLdsMax)
                         return g_stackLdsWide;
                 else
                         return g_stackLds;
         }
         __device__ __forceinline__ void put(int sp, int v) {
                 if (kLds > 0 && sp < kLds)
-                        rows()[sp * kBlock + threadIdx.x] = v;
+                        rows()[sp * kWidth + threadIdx.x] = v;
                 else
                         priv[sp - kLds] = v;
         }
@@ -221,7 +257,7 @@ struct Stack {
                 // The volatile LDS read keeps the two loads apart: merged, they become one generic
                 // (flat) load that pays the latency of both memories on every pop.
                 typedef __attribute__((address_space(3))) volatile int LdsInt;
-                if (kLds > 0 && sp < kLds) return *(LdsInt *)&rows()[sp * kBlock + threadIdx.x];
+                if (kLds > 0 && sp < kLds) return *(LdsInt *)&rows()[sp * kWidth + threadIdx.x];
                 return priv[sp - kLds];
         }
 };
@@ -239,9 +275,12 @@ enum : int { kStepGo = 0, kStepDone = 1, kStepOverflow = 2 };
 // 327K-triangle displaced sphere: 30.2 -> 25.4 ms; Cornell 512^2 x 16 spp: 3.60 -> 3.01 ms; 100K any-hit
 // rays on 200K triangles: 538 -> 508 us; 16M incoherent rays: 15.4 -> 14.9 ms. Letting lanes wait at a
 // leaf until 8 or 16 of the wave stand at one was slower (16M rays by 5%, 100K rays by 19% and 35%).
-template <bool kAny, bool kStats, int kLds>
-__device__ __forceinline__ int step(Lane &L, Stack<kLds> &S, const NodePair *__restrict__ nodes,
-                                    const TriRec *__restrict__ tris) {
+//
+// `boxes` (Scene::boxes) lets beyond_zero_axis cull; the path kernels pass 0, which takes that code out:
+// their rays have no zero component but for a measure-zero few, and its registers cost the megakernel 3%.
+template <bool kAny, bool kStats, int kLds, int kWidth = kBlock>
+__device__ __forceinline__ int step(Lane &L, Stack<kLds, kWidth> &S, const NodePair *__restrict__ nodes,
+                                    const TriRec *__restrict__ tris, int boxes = 0) {
         const float4 *rec = L.cur < 0 ? reinterpret_cast<const float4 *>(tris + ~L.cur)
                                       : reinterpret_cast<const float4 *>(nodes + L.cur);
         const float4 a = rec[0], b = rec[1], c = rec[2];
@@ -277,6 +316,10 @@ __device__ __forceinline__ int step(Lane &L, Stack<kLds> &S, const NodePair *__r
         } else {
                 lh = slab_exact(a.x, a.y, a.z, a.w, b.x, b.y, L.r, L.tBest, tl);
                 rh = slab_exact(b.z, b.w, c.x, c.y, c.z, c.w, L.r, L.tBest, tr);
+                if (!kStats && boxes == (kBoxesBounded | kBoxesNested)) {  // the counting kernels count the reference's visits
+                        lh = lh && !beyond_zero_axis(a.x, a.y, a.z, a.w, b.x, b.y, L.r);
+                        rh = rh && !beyond_zero_axis(b.z, b.w, c.x, c.y, c.z, c.w, L.r);
+                }
         }
         const int dl = __float_as_int(d.x), dr = __float_as_int(d.y);
         if (lh && rh) {

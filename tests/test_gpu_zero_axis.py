@@ -1,0 +1,93 @@
+"""Rays with zero direction components against the CPU oracle.
+
+A ray that does not move along an axis is culled by boxes it cannot meet there, which the reference's slab
+test lets through: the hits have to stay the oracle's bit for bit, also where triangles are large against
+the scene (the cull's bound is then wider than the box) and where the caller's boxes do not hold their
+triangles (the cull is then off).
+"""
+import numpy as np
+import pytest
+
+from gonzales_amd import scenes
+from helpers import OracleView, random_rays, random_soup_hierarchy
+from test_gpu_traversal import _assert_hits_equal, _device_any, _device_closest
+
+pytestmark = pytest.mark.gpu
+
+
+def _zero_axis_rays(n, seed, bh, scale=1.0):
+    """Random rays, one or two direction components set to +0 or -0, a fifth with an origin coordinate on a
+    vertex's own."""
+    g = np.random.default_rng(seed)
+    rays, tmax = random_rays(n, seed, lo=-0.2 * scale, hi=1.2 * scale, tmax=(0.1 * scale, 4.0 * scale))
+    first = g.integers(0, 3, n)
+    other = np.where(g.random(n) < 0.3, (first + 1) % 3, first)
+    pts = np.concatenate([m.points[:, :3] for m in bh.scene.meshes])
+    on = g.random(n) < 0.2
+    for a, (o, d) in enumerate((("orgX", "dirX"), ("orgY", "dirY"), ("orgZ", "dirZ"))):
+        z = (first == a) | (other == a)
+        rays[d][z] = np.where(g.random(z.sum()) < 0.5, 0.0, -0.0)
+        w = z & on
+        rays[o][w] = pts[g.integers(0, len(pts), w.sum()), a]
+    return rays, tmax
+
+
+def test_zero_components_of_rays_that_are_not_finite(gpu):
+    """NaN, infinite and huge origins or directions beside a zero component: tri_test accepts a NaN, so no
+    box may be skipped."""
+    bh = random_soup_hierarchy(5000, 13, scale=0.05)
+    bh.upload_to_gpu()
+    rays, tmax = _zero_axis_rays(20_000, 14, bh)
+    g = np.random.default_rng(15)
+    odd = np.asarray([np.nan, np.inf, -np.inf, 1e30, -3e38, 1e13], np.float32)
+    for name in ("orgX", "orgY", "orgZ", "dirX", "dirY", "dirZ"):
+        at = (g.random(len(rays)) < 0.1) & (rays[name] != 0.0)
+        rays[name][at] = odd[g.integers(0, len(odd), at.sum())]
+    ref, _ = OracleView(bh).closest(rays, tmax)
+    hits, _ = _device_closest(bh, rays, tmax)
+    assert np.array_equal(hits["prim"] >= 0, ref["hit"].astype(bool))
+    finite = np.isfinite(ref["tHit"])
+    for f, r in (("t", "tHit"), ("u", "u"), ("v", "v")):
+        assert np.array_equal(np.isnan(hits[f]), np.isnan(ref[r]))
+        assert np.array_equal(hits[f][finite], ref[r][finite], equal_nan=True)
+    occ, _ = _device_any(bh, rays, tmax)
+    assert np.array_equal(occ, ref["hit"].astype(bool))
+    bh.free()
+
+
+@pytest.mark.parametrize("n_tris,size,scale", [(40, 1.0, 1.0), (3000, 0.3, 1.0), (50_000, 0.02, 1.0),
+                                               (20_000, 0.0005, 1.0), (5000, 30.0, 100.0)])
+def test_zero_components_match_the_oracle(gpu, n_tris, size, scale):
+    bh = random_soup_hierarchy(n_tris, n_tris, spread=scale, scale=size)
+    bh.upload_to_gpu()
+    rays, tmax = _zero_axis_rays(20_000, 5, bh, scale)
+    ref, ref_st = OracleView(bh).closest(rays, tmax, stats=True)
+    hits, _ = _device_closest(bh, rays, tmax)
+    _assert_hits_equal(hits, ref)
+    occ, _ = _device_any(bh, rays, tmax)
+    assert np.array_equal(occ, ref["hit"].astype(bool))
+    _, st = _device_closest(bh, rays, tmax, stats=True)  # the counting kernels count the reference's visits
+    assert st.tobytes() == ref_st.tobytes()
+    bh.free()
+
+
+def test_zero_components_in_axis_aligned_planes(gpu):
+    bh, _ = scenes.cornell_hierarchy()
+    bh.upload_to_gpu()
+    rays, tmax = _zero_axis_rays(20_000, 6, bh, 2.0)
+    ref, _ = OracleView(bh).closest(rays, tmax)
+    hits, _ = _device_closest(bh, rays, tmax)
+    _assert_hits_equal(hits, ref)
+    bh.free()
+
+
+def test_boxes_that_do_not_hold_their_triangles(gpu):
+    bh = random_soup_hierarchy(2000, 7, scale=0.2)
+    lo = bh.nodes["boundsMinZ"].copy()
+    bh.nodes["boundsMinZ"] = lo + 0.6 * (bh.nodes["boundsMaxZ"] - lo)
+    bh.upload_to_gpu()
+    rays, tmax = _zero_axis_rays(20_000, 8, bh)
+    ref, _ = OracleView(bh).closest(rays, tmax)
+    hits, _ = _device_closest(bh, rays, tmax)
+    _assert_hits_equal(hits, ref)
+    bh.free()
