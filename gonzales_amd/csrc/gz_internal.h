@@ -129,6 +129,7 @@ struct Scene {
 
         // Traversal launch configuration.
         GzTraceConfig traceConfig{3, 16, 32, 1, 128, 1 << 18, 0, 0};
+        bool traceConfigSet = false;  // false: smaller batches take a lane per ray, unbinned (trace_plain)
         int boxes = 0;  // what is known of the node boxes: kBoxesBounded | kBoxesNested
         int cuCount = 256;
 };

@@ -489,6 +489,7 @@ extern "C" int gz_gpu_set_trace_config(void *handle, const GzTraceConfig *config
         Scene *s = static_cast<Scene *>(handle);
         std::lock_guard<std::mutex> lock(s->mu);
         s->traceConfig = *config;
+        s->traceConfigSet = true;
         return GZ_OK;
 }
 

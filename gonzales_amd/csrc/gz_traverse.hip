@@ -40,25 +40,28 @@ __device__ __forceinline__ int64_t lane_start_sorted(Lane &L, const SortedRay *_
         return (int64_t)__float_as_uint(r.b.w);
 }
 
-// One lane per ray, one ray per lane.
+// One lane per ray, one wave per workgroup: the hardware hands out the waves, with no counter that all
+// of them hit, and a wave's slot and stack are free as soon as its own longest ray ends. `perWave` rays a
+// wave (wave_rays). Bound by the latency of a wave's longest chain of record loads, under which the
+// waves on the chip (8 per SIMD) hide each other.
 template <bool kAny, bool kStats, int kLds>
-__global__ __launch_bounds__(kBlock) void k_trace(const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris,
-                                                  int rootDesc, int boxes, const Ray_C *__restrict__ rays,
-                                                  const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
-                                                  uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats,
-                                                  int *__restrict__ err, const SortedRay *__restrict__ order) {
-        const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-        if (j >= n) return;
+__global__ __launch_bounds__(64) void k_trace(const NodePair *__restrict__ nodes, const TriRec *__restrict__ tris,
+                                              int rootDesc, int boxes, const Ray_C *__restrict__ rays,
+                                              const float *__restrict__ tMaxIn, int64_t n, GzHit *__restrict__ hits,
+                                              uint8_t *__restrict__ occ, GzTraceStats *__restrict__ stats,
+                                              int *__restrict__ err, const SortedRay *__restrict__ order, int perWave) {
+        const int64_t j = (int64_t)blockIdx.x * perWave + threadIdx.x;
+        if ((int)threadIdx.x >= perWave || j >= n) return;
         Lane L;
         int64_t i = j;
         if (order)
                 i = lane_start_sorted(L, order, j, rootDesc, boxes);
         else
                 lane_start(L, rays, tMaxIn, i, rootDesc, boxes);
-        Stack<kLds> S;
+        Stack<kLds, 64> S;
         int st;
         do {
-                st = step<kAny, kStats, kLds>(L, S, nodes, tris, boxes);
+                st = step<kAny, kStats, kLds, 64>(L, S, nodes, tris, boxes);
         } while (st == kStepGo);
         lane_finish<kAny, kStats>(L, i, st == kStepOverflow, hits, occ, stats, err);
 }
@@ -482,12 +485,33 @@ __global__ __launch_bounds__(kBlock) void k_expand(const GzHit *__restrict__ hit
 
 static inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
+// Whether a batch is traced by k_trace with its rays in the given order: while the caller has set no
+// launch configuration, below kPersistentMinRays rays. Persistent lanes keep more of a wave busy on long
+// incoherent rays, but refilling them from a wave's own reserve leaves a tail that only a large batch
+// hides, and binning costs two passes over the rays. A million-triangle soup, incoherent rays, k_trace /
+// binned persistent lanes in ms: 2^18 rays 0.58 / 1.03, 2^20 1.5 / 1.9, 2^21 2.7 / 3.1, 2^22 5.0 / 4.3, 2^23
+// 9.7 / 7.7, 2^24 19.1 / 14.3. Shorter rays: 1080p camera rays on 82K triangles 0.22 / 1.1, 1.5M rays
+// around 50K triangles 0.35 / 1.1.
+static constexpr int64_t kPersistentMinRays = 1 << 22;
+static bool trace_plain(const Scene *s, int64_t n) { return !s->traceConfigSet && n < kPersistentMinRays; }
+
+// Rays per wave of k_trace: 64, or 32 or 16 where that still makes at most 4096 waves (4 per SIMD). A
+// batch that small leaves SIMDs idle, and a wave's step is shorter with fewer lanes loading (200,000
+// triangles, 100,000 any-hit rays: 250 us at 64 a wave, 236 at 32, 262 at 16, 387 at 8; 100,000
+// triangles, 4096 rays: 133 at 64, 128 at 32, 124 at 16, 135 at 8).
+static int wave_rays(int64_t n) {
+        int per = 64;
+        while (per > 16 && n <= (int64_t)4096 * (per / 2)) per >>= 1;
+        return per;
+}
+
 template <bool kAny, bool kStats, int kLds>
 static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays, const float *d_tMax, int64_t n,
                            GzHit *d_hits, uint8_t *d_occ, GzTraceStats *d_stats, hipStream_t stream,
                            const SortedRay *order) {
         const GzTraceConfig &c = s->traceConfig;
-        if (c.persistent == 2) {
+        const int mode = trace_plain(s, n) ? 0 : c.persistent;
+        if (mode == 2) {
                 auto kern = k_trace_strided<kAny, kStats, kLds>;
                 int perCU = 0;
                 if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, kBlock, 0) != hipSuccess || perCU < 1)
@@ -496,7 +520,7 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                 const unsigned g = (unsigned)std::min<int64_t>(want, grid_for(n));
                 hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, stream, s->dNodes, s->dTris, s->rootDesc,
                                    s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, order);
-        } else if (c.persistent == 3) {
+        } else if (mode == 3) {
                 auto kern = k_trace_xcd<kAny, kStats, kLds>;
                 int perCU = 0;
                 if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, kBlock, 0) != hipSuccess || perCU < 1)
@@ -508,7 +532,7 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                                    s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats, slot.dErr, slot.dCounter,
                                    c.refillLanes > 0 && c.refillLanes <= 64 ? c.refillLanes : 16,
                                    c.chunk >= 1 && c.chunk <= 4096 ? c.chunk : 64, order);
-        } else if (c.persistent == 1) {
+        } else if (mode == 1) {
                 auto kern = k_trace_persistent<kAny, kStats, kLds>;
                 int perCU = 0;
                 if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, kBlock, 0) != hipSuccess || perCU < 1)
@@ -522,9 +546,10 @@ static void launch_variant(Scene *s, const StreamSlot &slot, const Ray_C *d_rays
                                    c.refillLanes > 0 && c.refillLanes <= 64 ? c.refillLanes : 16,
                                    c.chunk >= 1 && c.chunk <= 4096 ? c.chunk : 64, order);
         } else {
-                hipLaunchKernelGGL((k_trace<kAny, kStats, kLds>), dim3(grid_for(n)), dim3(kBlock), 0, stream, s->dNodes,
-                                   s->dTris, s->rootDesc, s->boxes, d_rays, d_tMax, n, d_hits, d_occ, d_stats,
-                                   slot.dErr, order);
+                const int per = wave_rays(n);
+                hipLaunchKernelGGL((k_trace<kAny, kStats, kLds>), dim3((unsigned)((n + per - 1) / per)), dim3(64), 0,
+                                   stream, s->dNodes, s->dTris, s->rootDesc, s->boxes, d_rays, d_tMax, n, d_hits, d_occ,
+                                   d_stats, slot.dErr, order, per);
         }
 }
 
@@ -585,7 +610,7 @@ static const SortedRay *bin_rays(Scene *s, StreamSlot *slot, const Ray_C *d_rays
                                  hipStream_t stream, bool &failed) {
         failed = false;
         const int32_t minRays = s->traceConfig.binMinRays;
-        if (minRays <= 0 || n < minRays || s->empty || s->rootDesc < 0 || n > 0xffffffffLL) return nullptr;
+        if (minRays <= 0 || n < minRays || trace_plain(s, n) || s->empty || s->rootDesc < 0 || n > 0xffffffffLL) return nullptr;
         uint32_t nBlocks, tiles;
         int64_t entries;
         const uint32_t per = bin_per(n);

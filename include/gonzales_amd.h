@@ -282,7 +282,8 @@ int gz_gpu_expand_hits_device(void *handle, const struct GzHit *d_hits, const fl
  *                 parts of the tree; each ray's result still goes to its own index. 0 = always in
  *                 the given order;
  *   recordTimes : 1 = record HIP events around the binning and the traversal kernel of each
- *                 launch, for gz_gpu_trace_times (0 = none). */
+ *                 launch, for gz_gpu_trace_times (0 = none).
+ * Until a configuration is set, batches below 2^22 rays run in mode 0 in the given order. */
 struct GzTraceConfig {
         int32_t persistent;
         int32_t ldsStack;

@@ -1,4 +1,4 @@
-"""Rays with zero direction components against the CPU oracle.
+"""Rays with zero direction components, and the launch rule of small batches, against the CPU oracle.
 
 A ray that does not move along an axis is culled by boxes it cannot meet there, which the reference's slab
 test lets through: the hits have to stay the oracle's bit for bit, also where triangles are large against
@@ -90,4 +90,29 @@ def test_boxes_that_do_not_hold_their_triangles(gpu):
     ref, _ = OracleView(bh).closest(rays, tmax)
     hits, _ = _device_closest(bh, rays, tmax)
     _assert_hits_equal(hits, ref)
+    bh.free()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65_535, 65_536, 65_537, 131_072, 131_073])
+def test_batches_at_the_edges_of_the_wave_sizes(gpu, n):
+    bh = random_soup_hierarchy(500, 9, scale=0.1)
+    bh.upload_to_gpu()
+    rays, tmax = random_rays(n, 10)
+    ref, _ = OracleView(bh).closest(rays, tmax)
+    hits, _ = _device_closest(bh, rays, tmax)
+    _assert_hits_equal(hits, ref)
+    occ, _ = _device_any(bh, rays, tmax)
+    assert np.array_equal(occ, ref["hit"].astype(bool))
+    bh.free()
+
+
+def test_default_rule_on_both_sides_of_its_line(gpu):
+    bh = random_soup_hierarchy(500, 11, scale=0.1)
+    bh.upload_to_gpu()
+    rays, tmax = random_rays(1 << 22, 12)
+    whole, _ = _device_closest(bh, rays, tmax)
+    part, _ = _device_closest(bh, rays[:-1], tmax[:-1])
+    assert whole[:-1].tobytes() == part.tobytes()
+    sel = slice(0, 50_000)
+    _assert_hits_equal(whole[sel], OracleView(bh).closest(rays[sel], tmax[sel])[0])
     bh.free()
