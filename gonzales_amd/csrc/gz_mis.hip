@@ -135,8 +135,7 @@ __device__ __forceinline__ void queue_loop(unsigned count, const int *__restrict
 
 // ---- Split wavefront: one trace kernel and two shade kernels per bounce level ----------------
 //
-// k_wf_trace: persistent lanes with refill trace the closest hit of every path of the level's
-// queue (idle lanes take new paths from the queue when `refill` of them are idle) and store it;
+// k_wf_rays<0> traces the closest hit of every path of the level's queue, a lane per path, and stores it;
 // k_wf_split sorts the paths by the BSDF their hit shades with into the diffuse queue (misses and
 // stopped paths too) or the queue of the other BSDFs. k_wf_shade<kAll> then runs the rest of the
 // bounce (bounce_rest) over one class queue: the diffuse kernel is the small one (4 waves/SIMD),
@@ -167,96 +166,6 @@ __global__ void k_wf_clear(WfLevel *ctl, int levels) {
                 unsigned *u = reinterpret_cast<unsigned *>(&z);
                 for (int j = 0; j < 16; ++j) u[j] = 0u;
                 ctl[k] = z;
-        }
-}
-
-template <bool kStats>
-__global__ __launch_bounds__(kBlock) void k_wf_trace(MisArgs a, const GzPath *__restrict__ paths, unsigned count,
-                                                     const int *__restrict__ qin, WfLevel *ctl, int level,
-                                                     GzHit *__restrict__ hits, int refill, unsigned chunk,
-                                                     uint32_t *__restrict__ stats) {
-        Stack<kLdsMax> S;
-        Lane L;
-        int cur = -1;       // path index in flight on this lane
-        bool done = false;  // this lane finished a path this step
-        unsigned resBase = 0, resCount = 0;
-        bool counterDone = false, exhausted = false;
-        const int laneId = (int)(threadIdx.x & 63);
-        const uint64_t below = laneId == 0 ? 0ull : (~0ull >> (64 - laneId));
-        WfLevel &lv = ctl[level];
-        const unsigned nin = qin ? lv.qn : count;
-        for (;;) {
-                if (!exhausted) {
-                        const uint64_t idle = __ballot(cur < 0);
-                        const int nIdle = __popcll(idle);
-                        if (nIdle >= refill || nIdle == 64) {
-                                const unsigned rank = (unsigned)__popcll(idle & below);
-                                const unsigned need = (unsigned)nIdle;
-                                unsigned fresh = 0, take = 0;
-                                if (resCount < need && !counterDone) {
-                                        take = need - resCount > chunk ? need - resCount : chunk;
-                                        const int leader = __ffsll((unsigned long long)idle) - 1;
-                                        if (laneId == leader) fresh = atomicAdd(&lv.qhead, take);
-                                        fresh = __shfl(fresh, leader);
-                                        if (fresh >= nin || nin - fresh <= take) counterDone = true;
-                                }
-                                if (cur < 0) {
-                                        unsigned mine = 0xffffffffu;
-                                        if (rank < resCount)
-                                                mine = resBase + rank;
-                                        else if (rank - resCount < take)
-                                                mine = fresh + (rank - resCount);
-                                        if (mine < nin) {
-                                                cur = qin ? qin[mine] : (int)mine;
-                                                const GzPath &p = paths[cur];
-                                                if (path_live(a, p)) {
-                                                        lane_init(L, p.ray, INFINITY, a.rootDesc, a.boxes);
-                                                        done = a.empty;  // no nodes: a miss, nothing to step
-                                                } else {
-                                                        L.hitPrim = -1;
-                                                        L.nInterior = L.nTris = 0;
-                                                        done = true;  // stopped: the shade kernel clears it
-                                                }
-                                        }
-                                }
-                                if (take > 0) {
-                                        const unsigned used = need - resCount;
-                                        resBase = fresh + used;
-                                        resCount = take - used;
-                                } else {
-                                        const unsigned used = need < resCount ? need : resCount;
-                                        resBase += used;
-                                        resCount -= used;
-                                }
-                                if (counterDone && (resCount == 0 || resBase >= nin)) exhausted = true;
-                        }
-                }
-                if (cur >= 0 && !done) {
-                        const int st = step<false, kStats, kLdsMax>(L, S, a.nodes, a.tris);
-                        if (st != kStepGo) {
-                                if (st == kStepOverflow) {
-                                        atomicOr(a.err, 1);
-                                        L.hitPrim = -1;
-                                }
-                                done = true;
-                        }
-                }
-                // a finished path: store its hit (sorted into the class queues by k_wf_split)
-                if (cur >= 0 && done) {
-                        GzHit h;
-                        h.prim = L.hitPrim;
-                        h.t = L.hitPrim >= 0 ? L.tBest : INFINITY;
-                        h.u = L.hitPrim >= 0 ? L.bu : 0.0f;
-                        h.v = L.hitPrim >= 0 ? L.bv : 0.0f;
-                        hits[cur] = h;
-                        if (kStats) {
-                                stats[3 * (size_t)cur] += L.nInterior;
-                                stats[3 * (size_t)cur + 1] += L.nTris;
-                        }
-                        cur = -1;
-                        done = false;
-                }
-                if (exhausted && __ballot(cur >= 0) == 0ull) break;
         }
 }
 
@@ -456,33 +365,29 @@ __global__ __launch_bounds__(kMisBlock, kAll == kBsdfAll ? 2 : 3) void k_mis_adj
 
 // ---- Full wavefront: every ray of a bounce traced by a traversal kernel -------------------------
 //
-// Per level: k_wf_trace (closest hits of the paths' rays), k_wf_split (class queues), then per
+// Per level: k_wf_rays<0> (closest hits of the paths' rays), k_wf_split (class queues), then per
 // class k_wf_phase (shade_phase: the bounce up to its shadow and BSDF rays, which it appends to
 // two ray queues, and the continuation), k_wf_rays<1> and <2> (any hit of the shadow rays,
 // closest hit of the BSDF rays, 7 to 8 waves per SIMD) and k_wf_finish over the class queues
 // (finish_phase). The shade kernels trace nothing, so every traversal runs at the traversal
 // kernels' occupancy.
 
-// The rays of a queue of path indices, 64 per wave and chunk by static striding (no atomic),
-// each lane tracing its ray to the end: kMode 0 the paths' own rays (queue of level `level`, the
-// identity over `count` at level 0; stopped paths get a miss) into hits, 1 the shadow rays
-// `rays[i]` (any hit below 1 - 1e-5) into occ, 2 the BSDF rays (closest hit) into hits. On the
-// 5M-triangle frame, per 8M-path batch: shadow rays 2.7 ms here against 4.1 ms with k_wf_trace's
-// lane refill, BSDF rays 2.8 against 3.1 ms, but the paths' own rays 7.8 against 6.4 ms; so
-// k_wf_trace takes those.
+// The rays of a queue of path indices, one per lane, 64 to a one-wave workgroup, each lane tracing its
+// ray to the end: kMode 0 the paths' own rays (queue of level `level`, the identity over `count` at
+// level 0; stopped paths get a miss) into hits, 1 the shadow rays `rays[i]` (any hit below 1 - 1e-5)
+// into occ, 2 the BSDF rays (closest hit) into hits. One wave per workgroup, handed out by the hardware:
+// with persistent lanes that refilled from the queue the path rays' kernel (mode 0 now) took 1.96 times as
+// long on the 256^2 x 16 spp inverse-rendering frame (2.12 -> 1.07 ms of its 5.8 -> 4.7 ms); with 256-lane
+// groups by static striding the shadow rays took 7% longer. Bound by the chain of record loads.
 template <int kMode, bool kStats>
-__global__ __launch_bounds__(kBlock) void k_wf_rays(MisArgs a, const GzPath *__restrict__ paths, unsigned count,
-                                                    const int *__restrict__ qin, const unsigned *nptr,
-                                                    const Ray_C *__restrict__ rays, uint8_t *__restrict__ occ,
-                                                    GzHit *__restrict__ hits, uint32_t *__restrict__ stats) {
+__global__ __launch_bounds__(64) void k_wf_rays(MisArgs a, const GzPath *__restrict__ paths, unsigned count,
+                                                const int *__restrict__ qin, const unsigned *nptr,
+                                                const Ray_C *__restrict__ rays, uint8_t *__restrict__ occ,
+                                                GzHit *__restrict__ hits, uint32_t *__restrict__ stats) {
         constexpr bool kAny = kMode == 1;
-        Stack<kLdsMax> S;
+        Stack<kLdsMax, 64> S;
         const unsigned nin = (kMode == 0 && !qin) ? count : *nptr;
-        const int lane = (int)(threadIdx.x & 63);
-        const unsigned waves = gridDim.x * (blockDim.x >> 6);
-        for (unsigned g = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); (size_t)g * 64 < nin; g += waves) {
-                const unsigned j = g * 64 + (unsigned)lane;
-                if (j >= nin) continue;
+        for (size_t j = (size_t)blockIdx.x * 64 + threadIdx.x; j < nin; j += (size_t)gridDim.x * 64) {
                 const int idx = qin ? qin[j] : (int)j;
                 Lane L;
                 L.hitPrim = -1;
@@ -500,7 +405,7 @@ __global__ __launch_bounds__(kBlock) void k_wf_rays(MisArgs a, const GzPath *__r
                         const float tStop = kMode == 2 ? bsdf_ray_stop(a, rays[idx]) : -1.0f;
                         int st;
                         do {
-                                st = step<kAny, kStats, kLdsMax>(L, S, a.nodes, a.tris);
+                                st = step<kAny, kStats, kLdsMax, 64>(L, S, a.nodes, a.tris);
                         } while (st == kStepGo && !(kMode == 2 && L.hitPrim >= 0 && L.left == 0 && L.tBest < tStop));
                         if (st == kStepOverflow) {
                                 atomicOr(a.err, 1);
@@ -699,6 +604,12 @@ static unsigned queue_grid(Scene *s, K kern, int block, int64_t count, unsigned 
         const int64_t wavesPerBlock = block / 64;
         const int64_t need = ((count + chunk - 1) / chunk + wavesPerBlock - 1) / wavesPerBlock;
         return (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, need));
+}
+
+// Grid of k_wf_rays: a wave for every 64 entries the queue can hold, at most 256 a CU (a queue's length is
+// known to the device alone, and the waves past it only start and end).
+static unsigned rays_grid(const Scene *s, int64_t count) {
+        return (unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)s->cuCount * 256, (count + 63) / 64));
 }
 
 // Grid of k_wf_split: up to 8 blocks per CU, no more than the first level has tiles.
@@ -1171,10 +1082,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 MisQueue *q = full_queue(owner, st, (size_t)count, levels);
                 if (!q) return GZ_E_ALLOC;
                 const GzMisLaunch &c = s->misLaunch;
-                const GzTraceConfig &tc = s->traceConfig;
-                const int refill = tc.refillLanes > 0 && tc.refillLanes <= 64 ? tc.refillLanes : 56;
-                const unsigned tchunk = (unsigned)(tc.chunk >= 1 && tc.chunk <= 4096 ? tc.chunk : 64);
-                auto ktrace = d_stats ? k_wf_trace<true> : k_wf_trace<false>;
+                auto ktrace = d_stats ? k_wf_rays<0, true> : k_wf_rays<0, false>;
                 auto kany = d_stats ? k_wf_rays<1, true> : k_wf_rays<1, false>;
                 auto kclose = d_stats ? k_wf_rays<2, true> : k_wf_rays<2, false>;
                 auto kd = d_stats ? k_wf_phase<true, kBsdfDiffuse> : k_wf_phase<false, kBsdfDiffuse>;
@@ -1184,15 +1092,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 // the latter shade at 3 waves per SIMD instead of 2
                 const bool layered = s->mis->anyLayered, other = s->mis->anyOther;
                 const int classes = !all ? 1 : 3;
-                auto tgrid_of = [&](auto kern) {
-                        int perCU = 0;
-                        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, kBlock, 0) != hipSuccess ||
-                            perCU < 1)
-                                perCU = 1;
-                        return (unsigned)std::max<int64_t>(
-                                1, std::min<int64_t>((int64_t)s->cuCount * perCU * c.gridScale, (count + kBlock - 1) / kBlock));
-                };
-                const unsigned tgrid = tgrid_of(ktrace), agrid = tgrid_of(kany), cgrid = tgrid_of(kclose);
+                const unsigned tgrid = rays_grid(s, count);
                 const unsigned chunk = (unsigned)c.chunk;
                 const unsigned gd = queue_grid(s, kd, c.block, count, chunk);
                 const unsigned ga = queue_grid(s, ka, c.block, count, chunk);
@@ -1219,8 +1119,8 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                                                    &lv->qhead, chunk, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
-                        hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(kBlock), 0, st, a, d_paths, (unsigned)count, qin,
-                                           q->wctl, level, hits, refill, tchunk, stats);
+                        hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin, &lv->qn,
+                                           nullptr, nullptr, hits, stats);
                         hipLaunchKernelGGL(k_wf_split, dim3(spgrid), dim3(kMisBlock), 0, st, a, (unsigned)count, qin,
                                            q->wctl, level, hits, q->qd, q->qa, q->qn, classes);
                         hipLaunchKernelGGL(kd, dim3(gd), dim3(c.block), 0, st, a, d_paths, hits, q->qd, q->wctl, level,
@@ -1231,9 +1131,9 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                         if (all && other)
                                 hipLaunchKernelGGL(kn, dim3(gn), dim3(c.block), 0, st, a, d_paths, hits, q->qn, q->wctl,
                                                    level, qout, q->qs, q->qm, q->pend, q->srays, q->mrays, chunk, stats);
-                        hipLaunchKernelGGL(kany, dim3(agrid), dim3(kBlock), 0, st, a, d_paths, (unsigned)count, q->qs,
+                        hipLaunchKernelGGL(kany, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, q->qs,
                                            &lv->sn, q->srays, occ, nullptr, stats);
-                        hipLaunchKernelGGL(kclose, dim3(cgrid), dim3(kBlock), 0, st, a, d_paths, (unsigned)count, q->qm,
+                        hipLaunchKernelGGL(kclose, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, q->qm,
                                            &lv->mn, q->mrays, nullptr, mhits, stats);
                         hipLaunchKernelGGL(k_wf_finish, dim3(sgrid), dim3(kMisBlock), 0, st, a, d_paths, q->qd, &lv->dn,
                                            q->pend, occ, q->mrays, mhits);
@@ -1256,18 +1156,11 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 MisQueue *q = wf_queue(owner, st, (size_t)count, levels);
                 if (!q) return GZ_E_ALLOC;
                 const GzMisLaunch &c = s->misLaunch;
-                const GzTraceConfig &tc = s->traceConfig;
-                const int refill = tc.refillLanes > 0 && tc.refillLanes <= 64 ? tc.refillLanes : 56;
-                const unsigned tchunk = (unsigned)(tc.chunk >= 1 && tc.chunk <= 4096 ? tc.chunk : 64);
-                auto ktrace = d_stats ? k_wf_trace<true> : k_wf_trace<false>;
+                auto ktrace = d_stats ? k_wf_rays<0, true> : k_wf_rays<0, false>;
                 auto kd = d_stats ? k_wf_shade<true, 0> : k_wf_shade<false, 0>;
                 auto ka = d_stats ? (bset == kBsdfNoLayer ? k_wf_shade<true, 2> : k_wf_shade<true, 1>)
                                   : (bset == kBsdfNoLayer ? k_wf_shade<false, 2> : k_wf_shade<false, 1>);
-                int perCU = 0;
-                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, ktrace, kBlock, 0) != hipSuccess || perCU < 1)
-                        perCU = 1;
-                const unsigned tgrid = (unsigned)std::max<int64_t>(
-                        1, std::min<int64_t>((int64_t)s->cuCount * perCU * c.gridScale, (count + kBlock - 1) / kBlock));
+                const unsigned tgrid = rays_grid(s, count);
                 const unsigned chunk = (unsigned)c.chunk;
                 const unsigned gd = queue_grid(s, kd, c.block, count, chunk);
                 const unsigned ga = queue_grid(s, ka, c.block, count, chunk);
@@ -1283,8 +1176,8 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                                                    &q->wctl[level].qn, &q->wctl[level].qhead, chunk, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
-                        hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(kBlock), 0, st, a, d_paths, (unsigned)count, qin,
-                                           q->wctl, level, q->hits, refill, tchunk, stats);
+                        hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
+                                           &q->wctl[level].qn, nullptr, nullptr, q->hits, stats);
                         hipLaunchKernelGGL(k_wf_split, dim3(split_grid(s, count)), dim3(kMisBlock), 0, st, a,
                                            (unsigned)count, qin, q->wctl, level, q->hits, q->qd, q->qa, q->qa,
                                            all ? 2 : 1);
