@@ -46,7 +46,7 @@ __global__ __launch_bounds__(kMisBlock) void k_mis_adjoint(MisArgs a, GzPath *__
 // ---- Device path queues --------------------------------------------------------------------
 //
 // Bounce b of a trace runs over the queue of the paths still active after bounce b - 1 (bounce 0
-// over all paths). A persistent wave takes `chunk` queue entries per atomic on the level's head,
+// over all paths). A wave, a workgroup of its own, takes `chunk` queue entries,
 // bounces them 64 at a time, and appends the survivors to the next level's queue: a ballot of
 // the lanes that go on, a prefix popcount for each lane's slot and one atomic per wave for the
 // base. A wave's survivors keep their relative order, so neighbouring pixels stay together.
@@ -261,45 +261,35 @@ __global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_wf_shade(Mis
                                   return false;
                           }
                           const GzHit h = hits[i];
-                          Work w;
+                          Work<> w;
                           return bounce_rest<kStats, kAll, false>(a, paths, i, p, h.prim >= 0, h.prim, h.u, h.v, w,
                                                                   stats, AdjArgs{nullptr, nullptr}, nullptr);
                   });
 }
 
 template <bool kStats, int kAll>
-__global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_mis_queue(MisArgs a, GzPath *__restrict__ paths, unsigned count,
+__global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_mis_queue(MisArgs a, GzPath *__restrict__ paths, unsigned count,
                                                          const int *__restrict__ qin, int *__restrict__ qout,
                                                          QueueLevel *ctl, int level, unsigned chunk,
                                                          uint32_t *__restrict__ stats) {
-        queue_loop(count, qin, qout, ctl, level, chunk, [&](int i) {
-                return bounce_one<kStats, kAll, false>(a, paths, i, stats, AdjArgs{nullptr, nullptr}, nullptr);
+        queue_run(qin ? ctl[level].n : count, qin, nullptr, qout, &ctl[level + 1].n, chunk, [&](int i) {
+                return bounce_one<kStats, kAll, false, 64>(a, paths, i, stats, AdjArgs{nullptr, nullptr}, nullptr);
         });
 }
 
-// The remaining bounces of every path of one level's queue in one launch: a lane runs its path's
-// bounces until it stops (bounce_one returns false once the path is inactive or past maxDepth, so
-// at most maxDepth + 1 of them). For the last levels, where the few paths that Russian roulette
-// leaves cost less than one launch sequence per level.
+// The remaining bounces of every path of one level's queue (of all `count` paths at level 0) in one launch:
+// a lane runs its path's bounces until it stops (bounce_one returns false once the path is inactive or past
+// maxDepth, so at most maxDepth + 1 of them). For the last levels, where the few paths that Russian
+// roulette leaves cost less than one launch sequence per level.
 template <bool kStats, int kAll>
-__global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_mis_drain(MisArgs a, GzPath *__restrict__ paths,
-                                                                       const int *__restrict__ qin, const unsigned *nptr,
-                                                                       unsigned *head, unsigned chunk,
-                                                                       uint32_t *__restrict__ stats) {
-        const unsigned nin = *nptr;
-        const int lane = (int)(threadIdx.x & 63);
-        for (;;) {
-                unsigned c = 0;
-                if (lane == 0) c = atomicAdd(head, chunk);
-                c = __shfl(c, 0);
-                if (c >= nin) break;
-                const unsigned end = nin - c < chunk ? nin : c + chunk;
-                for (unsigned j = c + (unsigned)lane; j < end; j += 64) {
-                        const int i = qin[j];
-                        for (int b = 0; b <= a.maxDepth; ++b)
-                                if (!bounce_one<kStats, kAll, false>(a, paths, i, stats, AdjArgs{nullptr, nullptr}, nullptr))
-                                        break;
-                }
+__global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_mis_drain(MisArgs a, GzPath *__restrict__ paths, unsigned count,
+                                                                const int *__restrict__ qin, const unsigned *nptr,
+                                                                uint32_t *__restrict__ stats) {
+        const unsigned nin = qin ? *nptr : count;
+        for (size_t j = (size_t)blockIdx.x * 64 + threadIdx.x; j < nin; j += (size_t)gridDim.x * 64) {
+                const int i = qin ? qin[j] : (int)j;
+                for (int b = 0; b <= a.maxDepth; ++b)
+                        if (!bounce_one<kStats, kAll, false, 64>(a, paths, i, stats, AdjArgs{nullptr, nullptr}, nullptr)) break;
         }
 }
 
@@ -1019,6 +1009,33 @@ static void refresh_default_launch(Scene *s) {
                                             : GzMisLaunch{1, 256, 1, 256, 3, {0, 0, 0}};
 }
 
+// The launch a trace of `count` paths takes: the handle's, once gz_gpu_set_mis_launch has set one; else the
+// default by size. Small batches run whole: one launch, a lane per path through all its bounces
+// (k_mis_drain), since levels of a few hundred waves each wait out their longest path, and their launches
+// and queue counters cost more than the lanes that idle in a wave until its last path ends. The Cornell
+// box at depth 5 (four levels of queues and a drain before, with 256-lane groups / whole): 30K paths 0.87
+// -> 0.24 ms, 262K 0.93 -> 0.34; at 1M paths whole paths take 0.97 ms and levels of one-wave workgroups
+// 0.85, 3.1M 2.3 and 1.85, so those keep levels, with 128 entries a wave (64: 0.94 and 1.92 ms, 256: 0.85 and
+// 1.92). Scenes whose default is the wavefront, wavefront / whole: 120K paths on a 20K-triangle sphere 2.66 /
+// 1.42, 256K on 200K triangles 3.57 / 1.73, 1M on 300K 5.5 / 4.3 and on a 60K-triangle soup 1.9 / 1.0, 2.9M on
+// 300K 8.3 / 13.7: whole up to 2^20. A trace that keeps a record for the replay runs the levels it records.
+struct LaunchChoice {
+        GzMisLaunch launch;
+        bool wholePaths;
+};
+constexpr int64_t kWholePathsMega = 1 << 19, kWholePathsWavefront = 1 << 20;
+
+static LaunchChoice launch_for(const Scene *s, int64_t count, bool recording) {
+        LaunchChoice c{s->misLaunch, false};
+        if (s->misLaunchSet || recording) return c;
+        c.wholePaths = count <= (c.launch.queued == 3 ? kWholePathsWavefront : kWholePathsMega);
+        if (c.wholePaths)
+                c.launch.queued = 1;
+        else if (c.launch.queued == 1)
+                c.launch.chunk = 128;
+        return c;
+}
+
 constexpr int kMaxRecordLevels = 1025;  // maxDepth + 1 for the largest maxDepth (1024)
 
 // The three arrays of a replay record of `levels` levels of `count` paths at `base`.
@@ -1073,7 +1090,8 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
         uint32_t *stats = reinterpret_cast<uint32_t *>(d_stats);
         const bool all = !s->mis->allDiffuse;
         const int bset = mis_bsdf_set(s);
-        if (toEnd && s->misLaunch.queued == 3) {
+        const LaunchChoice lc = launch_for(s, count, rec != nullptr);
+        if (toEnd && lc.launch.queued == 3) {
                 if (count > 0x7fffffffLL) {
                         set_error("%s: %lld paths exceed one queue (2^31 - 1)", who, (long long)count);
                         return GZ_E_INVALID;
@@ -1102,7 +1120,6 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 const unsigned spgrid = split_grid(s, count);
                 auto kdrain = d_stats ? pick_set(bset, k_mis_drain<true, 0>, k_mis_drain<true, 1>, k_mis_drain<true, 2>)
                                       : pick_set(bset, k_mis_drain<false, 0>, k_mis_drain<false, 1>, k_mis_drain<false, 2>);
-                const unsigned gdrain = queue_grid(s, kdrain, c.block, count, chunk);
                 hipLaunchKernelGGL(k_wf_clear, dim3(1), dim3(256), 0, st, q->wctl, levels);
                 for (int level = 0; level <= params->maxDepth; ++level) {
                         const int *qin = level == 0 ? nullptr : q->q[level & 1];
@@ -1115,8 +1132,8 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                         GzHit *mhits = keep ? rec->mhits + (size_t)level * (size_t)count : q->mhits;
                         uint8_t *occ = keep ? rec->occ + (size_t)level * (size_t)count : q->occ;
                         if (c.drainLevel > 0 && level >= c.drainLevel) {
-                                hipLaunchKernelGGL(kdrain, dim3(gdrain), dim3(c.block), 0, st, a, d_paths, qin, &lv->qn,
-                                                   &lv->qhead, chunk, stats);
+                                hipLaunchKernelGGL(kdrain, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
+                                                   &lv->qn, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
                         hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin, &lv->qn,
@@ -1147,7 +1164,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 }
                 return GZ_OK;
         }
-        if (toEnd && s->misLaunch.queued == 2) {
+        if (toEnd && lc.launch.queued == 2) {
                 if (count > 0x7fffffffLL) {
                         set_error("%s: %lld paths exceed one queue (2^31 - 1)", who, (long long)count);
                         return GZ_E_INVALID;
@@ -1166,14 +1183,13 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 const unsigned ga = queue_grid(s, ka, c.block, count, chunk);
                 auto kdrain = d_stats ? pick_set(bset, k_mis_drain<true, 0>, k_mis_drain<true, 1>, k_mis_drain<true, 2>)
                                       : pick_set(bset, k_mis_drain<false, 0>, k_mis_drain<false, 1>, k_mis_drain<false, 2>);
-                const unsigned gdrain = queue_grid(s, kdrain, c.block, count, chunk);
                 hipLaunchKernelGGL(k_wf_clear, dim3(1), dim3(256), 0, st, q->wctl, levels);
                 for (int level = 0; level <= params->maxDepth; ++level) {
                         const int *qin = level == 0 ? nullptr : q->q[level & 1];
                         int *qout = q->q[(level + 1) & 1];
                         if (c.drainLevel > 0 && level >= c.drainLevel) {
-                                hipLaunchKernelGGL(kdrain, dim3(gdrain), dim3(c.block), 0, st, a, d_paths, qin,
-                                                   &q->wctl[level].qn, &q->wctl[level].qhead, chunk, stats);
+                                hipLaunchKernelGGL(kdrain, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
+                                                   &q->wctl[level].qn, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
                         hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
@@ -1190,7 +1206,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 }
                 return GZ_OK;
         }
-        if (toEnd && s->misLaunch.queued) {
+        if (toEnd && lc.launch.queued) {
                 if (count > 0x7fffffffLL) {
                         set_error("%s: %lld paths exceed one queue (2^31 - 1)", who, (long long)count);
                         return GZ_E_INVALID;
@@ -1199,20 +1215,29 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                                     : pick_set(bset, k_mis_queue<false, 0>, k_mis_queue<false, 1>, k_mis_queue<false, 2>);
                 auto kdrain = d_stats ? pick_set(bset, k_mis_drain<true, 0>, k_mis_drain<true, 1>, k_mis_drain<true, 2>)
                                       : pick_set(bset, k_mis_drain<false, 0>, k_mis_drain<false, 1>, k_mis_drain<false, 2>);
-                const int block = s->misLaunch.block;
-                std::function<void(unsigned, const int *, unsigned *, unsigned *, unsigned)> drain;
-                if (s->misLaunch.drainLevel > 0)
-                        drain = [&](unsigned grid, const int *qin, unsigned *n, unsigned *head, unsigned chunk) {
-                                hipLaunchKernelGGL(kdrain, dim3(grid), dim3(block), 0, st, a, d_paths, qin, n, head, chunk,
-                                                   stats);
-                        };
-                return queued_levels(
-                        s, owner, kern, count, params->maxDepth, st, who,
-                        [&](int level, unsigned grid, const int *qin, int *qout, QueueLevel *ctl, unsigned chunk) {
-                                hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, a, d_paths, (unsigned)count, qin,
-                                                   qout, ctl, level, chunk, stats);
-                        },
-                        drain);
+                if (lc.wholePaths) {
+                        hipLaunchKernelGGL(kdrain, dim3(rays_grid(s, count)), dim3(64), 0, st, a, d_paths, (unsigned)count,
+                                           nullptr, nullptr, stats);
+                        return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
+                }
+                const int levels = params->maxDepth + 2;
+                MisQueue *q = mis_queue(owner, st, (size_t)count, levels);
+                if (!q) return GZ_E_ALLOC;
+                const unsigned chunk = (unsigned)lc.launch.chunk;
+                const unsigned grid = (unsigned)std::max<int64_t>(
+                        1, std::min<int64_t>((int64_t)s->cuCount * 256, (count + chunk - 1) / chunk));
+                hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(256), 0, st, q->ctl, levels);
+                for (int level = 0; level <= params->maxDepth; ++level) {
+                        const int *qin = level == 0 ? nullptr : q->q[level & 1];
+                        if (lc.launch.drainLevel > 0 && level >= lc.launch.drainLevel) {
+                                hipLaunchKernelGGL(kdrain, dim3(rays_grid(s, count)), dim3(64), 0, st, a, d_paths,
+                                                   (unsigned)count, qin, &q->ctl[level].n, stats);
+                                break;
+                        }
+                        hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
+                                           q->q[(level + 1) & 1], q->ctl, level, chunk, stats);
+                }
+                return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
         }
         // A path makes at most maxDepth + 1 bounces (bounce 0 .. maxDepth); a launch after the
         // last finds every path inactive.

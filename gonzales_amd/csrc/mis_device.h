@@ -82,21 +82,22 @@ struct MisArgs {
 // and triangle tests, all rays).
 constexpr int kLdsMis = kLdsWide;
 
+template <int kWidth = kBlock>
 struct Work {
-        Stack<kLdsMis> S;
+        Stack<kLdsMis, kWidth> S;
         uint32_t interior = 0, tris = 0;
 };
 
 // Closest or any hit of one ray (the traversal of the batch kernels, inline).
-template <bool kAny, bool kStats>
+template <bool kAny, bool kStats, int kWidth>
 __device__ __forceinline__ bool trace_ray(const MisArgs &a, const Ray_C &ray, float tMax, int &prim, float &t,
-                                          float &u, float &v, Work &w) {
+                                          float &u, float &v, Work<kWidth> &w) {
         if (a.empty) return false;
         Lane L;
         lane_init(L, ray, tMax, a.rootDesc, a.boxes);
         int st;
         do {
-                st = step<kAny, kStats, kLdsMis>(L, w.S, a.nodes, a.tris);
+                st = step<kAny, kStats, kLdsMis, kWidth>(L, w.S, a.nodes, a.tris);
         } while (st == kStepGo);
         if (kStats) {
                 w.interior += L.nInterior;
@@ -139,15 +140,15 @@ __device__ __forceinline__ float bsdf_ray_stop(const MisArgs &a, const Ray_C &r)
 }
 
 // trace_ray's closest hit that stops once a hit closer than tStop is found (see bsdf_ray_stop).
-template <bool kStats>
+template <bool kStats, int kWidth>
 __device__ __forceinline__ bool trace_ray_until(const MisArgs &a, const Ray_C &ray, float tStop, int &prim, float &t,
-                                                float &u, float &v, Work &w) {
+                                                float &u, float &v, Work<kWidth> &w) {
         if (a.empty) return false;
         Lane L;
         lane_init(L, ray, INFINITY, a.rootDesc, a.boxes);
         int st;
         do {
-                st = step<false, kStats, kLdsMis>(L, w.S, a.nodes, a.tris);
+                st = step<false, kStats, kLdsMis, kWidth>(L, w.S, a.nodes, a.tris);
         } while (st == kStepGo && !(L.hitPrim >= 0 && L.left == 0 && L.tBest < tStop));
         if (kStats) {
                 w.interior += L.nInterior;
@@ -393,8 +394,8 @@ __device__ __forceinline__ void light_sample(const MisArgs &a, int choice, f3 po
 
 // Visibility.occluded via spawnRay(from:target:) (Visibility.swift:5-24, Interaction.swift:15-24):
 // origin from + 1e-4 (target - from), unnormalised direction, tMax 1 - 1e-5.
-template <bool kStats>
-__device__ __forceinline__ bool occluded(const MisArgs &a, f3 from, f3 target, Work &w) {
+template <bool kStats, int kWidth>
+__device__ __forceinline__ bool occluded(const MisArgs &a, f3 from, f3 target, Work<kWidth> &w) {
         const f3 o = add(from, mul(sub(target, from), 0.0001f));
         const f3 d = sub(target, o);
         Ray_C r{o.x, o.y, o.z, d.x, d.y, d.z};
@@ -575,9 +576,9 @@ __device__ __forceinline__ bool path_live(const MisArgs &a, const GzPath &p) {
 
 // The bounce of path i (record p, already loaded and live) after its closest hit: `traced` and
 // (prim, hu, hv) are the closest hit of p.ray. Returns whether the path goes on.
-template <bool kStats, int kAll, bool kAdj>
+template <bool kStats, int kAll, bool kAdj, int kWidth>
 __device__ __forceinline__ bool bounce_rest(const MisArgs &a, GzPath *__restrict__ paths, int64_t i, GzPath p,
-                                            bool traced, int prim, float hu, float hv, Work &w,
+                                            bool traced, int prim, float hu, float hv, Work<kWidth> &w,
                                             uint32_t *__restrict__ stats, const AdjArgs &adj, double *lds) {
         f3 T = mk(p.throughput[0], p.throughput[1], p.throughput[2]);
         f3 E = mk(p.estimate[0], p.estimate[1], p.estimate[2]);
@@ -935,7 +936,7 @@ __device__ __forceinline__ void finish_phase(const MisArgs &a, GzPath *__restric
 }
 
 // One bounce of path i; returns whether the path goes on to another bounce.
-template <bool kStats, int kAll, bool kAdj>
+template <bool kStats, int kAll, bool kAdj, int kWidth = kBlock>
 __device__ __forceinline__ bool bounce_one(const MisArgs &a, GzPath *__restrict__ paths, int64_t i,
                                            uint32_t *__restrict__ stats, const AdjArgs &adj, double *lds) {
         const GzPath p = paths[i];
@@ -944,7 +945,7 @@ __device__ __forceinline__ bool bounce_one(const MisArgs &a, GzPath *__restrict_
                 paths[i].flags = p.flags & ~GZ_PATH_ACTIVE;
                 return false;
         }
-        Work w;
+        Work<kWidth> w;
         int prim = -1;
         float th, hu = 0.0f, hv = 0.0f;
         bool traced;

@@ -231,16 +231,19 @@ constexpr int kLdsWide = 32;
 __shared__ int g_stackLds[kLdsMax * kBlock];
 __shared__ int g_stackLdsWide[kLdsWide * kBlock];
 __shared__ int g_stackLdsWave[kLdsMax * 64];
+__shared__ int g_stackLdsWideWave[kLdsWide * 64];
 
 // Traversal stack of GZ_STACK_CAPACITY entries: the first kLds live in LDS, the rest in
 // per-lane private memory.
 template <int kLds, int kWidth = kBlock>
 struct Stack {
         static_assert(kLds <= kLdsWide, "LDS stack rows");
-        static_assert(kWidth == kBlock || (kWidth == 64 && kLds <= kLdsMax), "LDS stack width");
+        static_assert(kWidth == kBlock || kWidth == 64, "LDS stack width");
         int priv[GZ_STACK_CAPACITY - kLds > 0 ? GZ_STACK_CAPACITY - kLds : 1];
         __device__ __forceinline__ static int *rows() {
-                if constexpr (kWidth == 64)
+                if constexpr (kWidth == 64 && kLds > kLdsMax)
+                        return g_stackLdsWideWave;
+                else if constexpr (kWidth == 64)
                         return g_stackLdsWave;
                 else if constexpr (kLds > kLdsMax)
                         return g_stackLdsWide;

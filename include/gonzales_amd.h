@@ -418,18 +418,19 @@ int gz_gpu_mis_trace_device(void *handle, struct GzPath *d_paths, int64_t count,
 
 /* Launch configuration of gz_gpu_mis_trace_device, _trace_stats_device and _adjoint_device
  * (results never depend on it; no counterpart in the reference):
- *   queued    : 1 = persistent waves over device path queues, compacted after every bounce by a
+ *   queued    : 1 = waves over device path queues, compacted after every bounce by a
  *               wave ballot and prefix popcount (one atomic per wave); 2 = the same queues with
- *               each bounce split in a closest-hit kernel (lanes refilled from the queue, hits
+ *               each bounce split in a closest-hit kernel (a lane per path, hits
  *               sorted by material class into two queues) and one shade kernel per class, the
  *               diffuse one small; 3 = the full wavefront: as 2, with the shade kernels tracing
  *               nothing (they queue each path's shadow ray and BSDF ray), an any-hit and a
  *               closest-hit kernel trace those two ray queues, and a finish kernel per class adds
  *               the two strategies' terms; 0 = every bounce launches one lane per path of all
  *               `count` (stopped paths idle in their waves). The adjoint replays queue 1 for 1-3;
- *   block     : threads per workgroup, 64, 128 or 256;
- *   gridScale : persistent grid = gridScale x the workgroups resident per CU x CUs (1..16);
- *   chunk     : queue entries a wave takes per atomic, a multiple of 64 in 64..4096;
+ *   block     : threads per workgroup of the shade kernels and the adjoint's, 64, 128 or 256 (the kernels
+ *               that trace run one wave per workgroup);
+ *   gridScale : their persistent grid = gridScale x the workgroups resident per CU x CUs (1..16);
+ *   chunk     : queue entries a wave takes at a time, a multiple of 64 in 64..4096;
  *   drainLevel: 0, or 1..64 with a queued mode: the paths left at that bounce level run all their
  *               remaining bounces in one launch (a lane per path), in place of one launch
  *               sequence per level for the few paths that Russian roulette leaves (the
@@ -437,7 +438,8 @@ int gz_gpu_mis_trace_device(void *handle, struct GzPath *d_paths, int64_t count,
  *   reserved  : zero.
  * Until gz_gpu_set_mis_launch sets one, a handle uses {1, 256, 1, 256, 3} if every material is
  * diffuse and it has at most 65536 primitives, else {3, 256, 1, 64, 3} (gz_gpu_get_mis_launch
- * returns the one in use). */
+ * returns the one in use); up to 2^19 paths (2^20 for the latter) a forward trace then runs each path
+ * whole, in one launch, and keeps no queues. */
 struct GzMisLaunch {
         int32_t queued;
         int32_t block;

@@ -1,0 +1,52 @@
+"""The default launch of a path trace on both sides of its size rules: records equal, byte for byte, to one
+launch per bounce over all paths (queued = 0)."""
+import numpy as np
+import pytest
+
+from gonzales_amd import abi
+from gonzales_amd.accelerator import BoundingHierarchy
+from gonzales_amd.camera import cornell_camera
+from gonzales_amd.integrator import (MisOptions, VolumePathIntegrator, coated_conductor_material, conductor_material,
+                                     dielectric_material, diffuse_material)
+from gonzales_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _integrator(diffuse):
+    bh, _ = scenes.cornell_hierarchy()
+    bh = BoundingHierarchy(bh.scene, bh.prim_ids, bh.nodes)
+    bh.upload_to_gpu()
+    cam = cornell_camera(res=512, spp=8, seed=3)
+    opt = MisOptions(max_depth=4, zsobol_seed=cam.c.zsSeed, log2_spp=cam.c.zsLog2Spp, base4_digits=cam.c.zsBase4Digits)
+    if diffuse:
+        return VolumePathIntegrator(bh, opt), cam
+    kinds = [diffuse_material((0.5, 0.4, 0.3)), dielectric_material(eta=1.5, roughness=0.2),
+             conductor_material(roughness=0.3), coated_conductor_material(interface_roughness=0.1, conductor_roughness=0.3)]
+    mats = abi.concat([kinds[k % 4] for k in range(len(bh.scene.materials))], abi.GZ_MATERIAL)
+    return VolumePathIntegrator(bh, opt, materials=mats), cam
+
+
+@pytest.mark.parametrize("diffuse,counts", [(True, (1, 63, 65, 4097, 1 << 19, (1 << 19) + 1)),
+                                            (False, (1, 65, 4097, 1 << 20, (1 << 20) + 1))])
+def test_default_launch_equals_the_full_relaunch(gpu, diffuse, counts):
+    import torch
+
+    integ, cam = _integrator(diffuse)
+    assert cam.path_count > max(counts)
+    got = []
+    for n in counts:
+        buf = torch.empty(n * abi.GZ_PATH.itemsize, dtype=torch.uint8, device="cuda")
+        cam.paths_device(buf, 0, n)
+        integ.trace(buf, n)
+        got.append(buf.cpu().numpy())
+    integ.bh.check_traversal()
+    integ.set_launch(0)
+    n = max(counts)
+    buf = torch.empty(n * abi.GZ_PATH.itemsize, dtype=torch.uint8, device="cuda")
+    cam.paths_device(buf, 0, n)
+    integ.trace(buf, n)
+    ref = buf.cpu().numpy()
+    for n, g in zip(counts, got):
+        assert np.array_equal(g, ref[:n * abi.GZ_PATH.itemsize]), n
+    integ.bh.free()
