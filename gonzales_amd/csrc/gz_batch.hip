@@ -9,7 +9,7 @@
 //   clear   the per-level, per-item queue counters (a kernel, no memset: graph-safe);
 //   per level 0 .. maxDepth:
 //     plan    one lane: each item's chunk count and their running sum;
-//     bounce  persistent waves take one chunk per atomic; a chunk belongs to one item, so the
+//     bounce  one-wave workgroups stride over the chunks; a chunk belongs to one item, so the
 //             wave's scene is uniform and its MisArgs come from the scene table by scalar loads;
 //             survivors go to the item's queue of the next level by ballot + prefix popcount;
 //   film    one lane per pixel: the pixel's samples into its scene's film, in sample order;
@@ -99,11 +99,10 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_camera(const int *__restr
         paths[t] = camera_path(cams[it.scene], table, it.first + (t - it.offset));
 }
 
-// Per level: n[level][item] queue entries, head[level] chunks handed out, base[level][item]
+// Per level: n[level][item] queue entries, base[level][item]
 // the chunk running sum (base[level][nItems] = the level's chunks).
 struct BatchCounters {
         unsigned *n;
-        unsigned *head;
         unsigned *base;
         int maxItems;
         int levels;
@@ -112,7 +111,6 @@ struct BatchCounters {
 __global__ void k_batch_clear(BatchCounters c) {
         const int nn = (c.levels + 1) * c.maxItems;
         for (int k = threadIdx.x; k < nn; k += blockDim.x) c.n[k] = 0u;
-        for (int k = threadIdx.x; k < c.levels; k += blockDim.x) c.head[k] = 0u;
 }
 
 // One lane: each item's chunk count at `level` and their running sum, into `base`. select -1
@@ -133,12 +131,12 @@ __global__ void k_batch_plan(const int *__restrict__ cursor, const BatchRound *_
         base[R.nItems] = sum;
 }
 
-// One bounce level of a round: waves take chunks of the level's work items through one global
-// counter; survivors go to the item's next-level queue (appends held over four runs of 64 and
+// One bounce level of a round: one-wave workgroups stride over the chunks of the level's work
+// items; survivors go to the item's next-level queue (appends held over four runs of 64 and
 // written with one atomic). kDrain: a lane runs each path's remaining bounces instead, and no
 // queue is written (the last levels of a round, in one launch).
 template <int kAll, bool kDrain>
-__global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_batch_bounce(const int *__restrict__ cursor,
+__global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_batch_bounce(const int *__restrict__ cursor,
                                                             const BatchRound *__restrict__ rounds,
                                                             const BatchItem *__restrict__ items,
                                                             const MisArgs *__restrict__ args, GzPath *__restrict__ paths,
@@ -152,11 +150,7 @@ __global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_batch_bounce
         const unsigned *nIn = c.n + (size_t)level * c.maxItems;
         const int lane = (int)(threadIdx.x & 63);
         const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-        for (;;) {
-                unsigned g = 0;
-                if (lane == 0) g = atomicAdd(&c.head[level], 1u);
-                g = (unsigned)__builtin_amdgcn_readfirstlane((int)__shfl(g, 0));
-                if (g >= total) break;
+        for (unsigned g = blockIdx.x; g < total; g += gridDim.x) {
                 const int k = __builtin_amdgcn_readfirstlane(
                         find_item(R.nItems, (int)g, [&](int i) { return (int)base[i]; }));
                 const BatchItem it = its[k];
@@ -168,8 +162,8 @@ __global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_batch_bounce
                         for (unsigned j = e0 + (unsigned)lane; j < e1; j += 64) {
                                 const int idx = level == 0 ? it.offset + (int)j : qin[it.offset + (int)j];
                                 for (int b = 0; b <= a.maxDepth; ++b)
-                                        if (!bounce_one<false, kAll, false>(a, paths, idx, nullptr, AdjArgs{nullptr, nullptr},
-                                                                           nullptr))
+                                        if (!bounce_one<false, kAll, false, 64>(a, paths, idx, nullptr, AdjArgs{nullptr, nullptr},
+                                                                               nullptr))
                                                 break;
                         }
                         continue;
@@ -183,8 +177,8 @@ __global__ __launch_bounds__(kMisBlock, mis_min_waves(kAll)) void k_batch_bounce
                         const unsigned j = j0 + (unsigned)lane;
                         int idx = -1;
                         if (j < e1) idx = level == 0 ? it.offset + (int)j : qin[it.offset + (int)j];
-                        const bool go = idx >= 0 && bounce_one<false, kAll, false>(a, paths, idx, nullptr,
-                                                                                   AdjArgs{nullptr, nullptr}, nullptr);
+                        const bool go = idx >= 0 && bounce_one<false, kAll, false, 64>(a, paths, idx, nullptr,
+                                                                                       AdjArgs{nullptr, nullptr}, nullptr);
                         keep.set(runs, idx);
                         bits[0] |= (go ? 1u : 0u) << runs;
                         if (++runs == 4) {
@@ -319,7 +313,7 @@ __device__ __forceinline__ bool next_chunk(const BatchRound &R, const unsigned *
 // kMode 0: the path rays of the level queue (closest hit into hits, paths that stop get a miss),
 // 1: the shadow rays (any hit below 1 - 1e-5 into occ), 2: the BSDF rays (closest hit into mhits).
 template <int kMode>
-__global__ __launch_bounds__(kMisBlock) void k_bw_rays(const int *__restrict__ cursor,
+__global__ __launch_bounds__(64) void k_bw_rays(const int *__restrict__ cursor,
                                                        const BatchRound *__restrict__ rounds,
                                                        const BatchItem *__restrict__ items,
                                                        const MisArgs *__restrict__ args,
@@ -327,7 +321,7 @@ __global__ __launch_bounds__(kMisBlock) void k_bw_rays(const int *__restrict__ c
                                                        const unsigned *__restrict__ base, const unsigned *__restrict__ nIn,
                                                        WaveSlots ws, int level) {
         constexpr bool kAny = kMode == 1;
-        Stack<kLdsMax> S;
+        Stack<kLdsMax, 64> S;
         const BatchRound R = rounds[cursor[0]];
         const BatchItem *its = items + R.firstItem;
         const int lane = (int)(threadIdx.x & 63);
@@ -335,7 +329,7 @@ __global__ __launch_bounds__(kMisBlock) void k_bw_rays(const int *__restrict__ c
         first_chunk(ch);
         for (;;) {
                 const unsigned g = (unsigned)__builtin_amdgcn_readfirstlane((int)ch.g);
-                ch.g = g + gridDim.x * (blockDim.x >> 6);
+                ch.g = g + gridDim.x;
                 if (g >= base[R.nItems]) break;
                 const int k = __builtin_amdgcn_readfirstlane(chunk_item(R, base, g, ch.k));
                 ch.k = k;
@@ -359,7 +353,7 @@ __global__ __launch_bounds__(kMisBlock) void k_bw_rays(const int *__restrict__ c
                         if (trace && !a.empty) {
                                 int st;
                                 do {
-                                        st = step<kAny, false, kLdsMax>(L, S, a.nodes, a.tris);
+                                        st = step<kAny, false, kLdsMax, 64>(L, S, a.nodes, a.tris);
                                 } while (st == kStepGo);
                                 if (st == kStepOverflow) {
                                         atomicOr(a.err, 1);
@@ -584,6 +578,7 @@ struct Batch {
         std::vector<BatchRound> hRounds;
         std::vector<BatchItem> hItems;
         GzMisLaunch launch{1, 256, 1, 256, 3, {0, 0, 0}};
+        bool wholePaths = false;  // a round is one launch, a lane per path through all its bounces
         int cuCount = 256;
 
         int *dCursor = nullptr;
@@ -594,7 +589,7 @@ struct Batch {
         BatchFilm *dFilms = nullptr;
         GzPath *dPaths = nullptr;
         int *dQ[2] = {nullptr, nullptr};
-        BatchCounters ctr{nullptr, nullptr, nullptr, 0, 0};
+        BatchCounters ctr{nullptr, nullptr, 0, 0};
         const uint32_t *sobol = nullptr;
         // wavefront rounds (allocated by the first launch shape that asks for them)
         WaveCounters wctr{nullptr, nullptr, 0, 0};
@@ -648,7 +643,7 @@ static void free_batch(Batch *b) {
         }
         if (b->fork) (void)hipEventDestroy(b->fork);
         void *ptrs[] = {b->dErr,      b->dCursor,   b->dRounds,  b->dItems,   b->dArgs,     b->dCams,     b->dFilms,
-                        b->dPaths,    b->dQ[0],    b->dQ[1],    b->ctr.n,     b->ctr.head,  b->ctr.base,
+                        b->dPaths,    b->dQ[0],    b->dQ[1],    b->ctr.n,     b->ctr.base,
                         b->wctr.n,    b->wctr.base, b->ws.hits,  b->ws.pend,   b->ws.srays,
                         b->ws.mrays,  b->ws.occ,   b->ws.mhits, b->ws.q[0],  b->ws.q[1],   b->ws.q[2],
                         b->ws.q[3]};
@@ -704,6 +699,10 @@ static bool upload(T **dst, const T *src, size_t count, const char *what) {
         return count == 0 || hip_ok(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice), what);
 }
 
+// Rounds of at most this many paths run whole under the default launch (with and without scenes that
+// default to the wavefront).
+constexpr int64_t kWholeRoundWavefront = 3 << 20, kWholeRoundMega = 1 << 19;
+
 // Enqueues one round's launch sequence on `st`.
 static bool enqueue_round(Batch *b, hipStream_t st) {
         const unsigned chunk = (unsigned)b->launch.chunk;
@@ -711,16 +710,29 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
         auto kern = pick_set(b->bsdfSet, k_batch_bounce<0, false>, k_batch_bounce<1, false>, k_batch_bounce<2, false>);
         auto kdrain = pick_set(b->bsdfSet, k_batch_bounce<0, true>, k_batch_bounce<1, true>, k_batch_bounce<2, true>);
         const int drainLevel = b->launch.drainLevel;
-        int perCU = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, block, 0) != hipSuccess || perCU < 1) perCU = 1;
-        const int64_t want = (int64_t)b->cuCount * perCU * b->launch.gridScale;
-        const int64_t need = ((int64_t)b->roundPaths + chunk - 1) / chunk * 64 / block + 1;
-        const unsigned grid = (unsigned)std::max<int64_t>(1, std::min(want, need));
+        // the kernels that trace: a one-wave workgroup per chunk the round can have (an item ends its last
+        // chunk early), at most 256 a CU; they stride over the rest
+        auto wave_grid = [&](int64_t entries) {
+                return (unsigned)std::min<int64_t>((int64_t)b->cuCount * 256,
+                                                   ((int64_t)b->roundPaths + entries - 1) / entries + b->maxItems);
+        };
+        const unsigned grid = wave_grid(chunk);
         const unsigned camBlocks = (unsigned)((b->roundPaths + kBatchBlock - 1) / kBatchBlock);
         const unsigned filmBlocks = (unsigned)((b->maxRoundPixels + kBatchBlock - 1) / kBatchBlock);
         hipLaunchKernelGGL(k_batch_camera, dim3(camBlocks), dim3(kBatchBlock), 0, st, b->dCursor, b->dRounds, b->dItems,
                            b->dCams, b->sobol, b->dPaths);
         hipLaunchKernelGGL(k_batch_clear, dim3(1), dim3(256), 0, st, b->ctr);
+        if (b->wholePaths) {
+                const unsigned per = wave_paths(b->roundPaths, b->bsdfSet);
+                hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(64), 0, st, b->dCursor, b->dRounds, b->dItems, b->ctr, 0, per,
+                                   b->ctr.base, -1);
+                hipLaunchKernelGGL(kdrain, dim3(wave_grid(per)), dim3(64), 0, st, b->dCursor, b->dRounds, b->dItems, b->dArgs,
+                                   b->dPaths, b->dQ[0], b->dQ[1], b->ctr, 0, per);
+                hipLaunchKernelGGL(k_batch_film, dim3(filmBlocks), dim3(kBatchBlock), 0, st, b->dCursor, b->dRounds,
+                                   b->dItems, b->dFilms, b->dPaths);
+                hipLaunchKernelGGL(k_batch_next, dim3(1), dim3(64), 0, st, b->dCursor);
+                return hip_ok(hipGetLastError(), "batch round launch");
+        }
         if (b->launch.queued == 3) {
                 hipLaunchKernelGGL(k_bw_clear, dim3(1), dim3(256), 0, st, b->wctr);
                 auto kd = k_bw_phase<kBsdfDiffuse>;
@@ -729,13 +741,11 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                 // least 256 entries (their work per entry is short next to the per-chunk item lookup
                 // and queue appends)
                 const unsigned pchunk = std::max(256u, chunk);
-                const unsigned gt = batch_grid(b, k_bw_rays<0>, block, 64u),
+                const unsigned gt = wave_grid(64),
                                gsplit = (unsigned)std::max<int64_t>(
                                        1, std::min<int64_t>((int64_t)b->cuCount * 8,
                                                             ((int64_t)b->roundPaths + kSplitTile - 1) / kSplitTile + 64)),
                                gd = batch_grid(b, kd, block, pchunk), ga = batch_grid(b, ka, block, pchunk),
-                               gany = batch_grid(b, k_bw_rays<1>, block, 64u),
-                               gclose = batch_grid(b, k_bw_rays<2>, block, 64u),
                                gfin = batch_grid(b, k_bw_finish, block, pchunk);
                 const int *c = b->dCursor;
                 for (int level = 0; level < b->levels; ++level) {
@@ -743,7 +753,7 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                         if (drainLevel > 0 && level >= drainLevel) {
                                 hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(64), 0, st, c, b->dRounds, b->dItems, b->ctr,
                                                    level, chunk, lbase, -1);
-                                hipLaunchKernelGGL(kdrain, dim3(grid), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
+                                hipLaunchKernelGGL(kdrain, dim3(grid), dim3(64), 0, st, c, b->dRounds, b->dItems, b->dArgs,
                                                    b->dPaths, b->dQ[level & 1], b->dQ[(level + 1) & 1], b->ctr, level,
                                                    chunk);
                                 break;
@@ -752,7 +762,7 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                         if (b->anyMega) {
                                 hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(64), 0, st, c, b->dRounds, b->dItems, b->ctr,
                                                    level, chunk, lbase, 0);
-                                hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
+                                hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, c, b->dRounds, b->dItems, b->dArgs,
                                                    b->dPaths, b->dQ[level & 1], b->dQ[(level + 1) & 1], b->ctr, level,
                                                    chunk);
                         }
@@ -762,7 +772,7 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                         hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(64), 0, st, c, b->dRounds, b->dItems, b->ctr, level,
                                            kSplitTile, b->wctr.baseOf(level, kWLevelSplit), 1);
                         const unsigned *nLevel = b->ctr.n + (size_t)level * b->ctr.maxItems;
-                        hipLaunchKernelGGL(k_bw_rays<0>, dim3(gt), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
+                        hipLaunchKernelGGL(k_bw_rays<0>, dim3(gt), dim3(64), 0, st, c, b->dRounds, b->dItems, b->dArgs,
                                            b->dPaths, b->dQ[level & 1], b->wctr.baseOf(level, kWLevel), nLevel, b->ws,
                                            level);
                         hipLaunchKernelGGL(k_bw_split, dim3(gsplit), dim3(kMisBlock), 0, st, c, b->dRounds, b->dItems,
@@ -776,10 +786,10 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                                                    b->dPaths, b->dQ[(level + 1) & 1], b->ctr, b->wctr, b->ws, level, pchunk);
                         hipLaunchKernelGGL(k_bw_plan, dim3(1), dim3(64), 0, st, c, b->dRounds, b->wctr, level,
                                            (1 << kWShadow) | (1 << kWBsdf), 64u);
-                        hipLaunchKernelGGL(k_bw_rays<1>, dim3(gany), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
+                        hipLaunchKernelGGL(k_bw_rays<1>, dim3(gt), dim3(64), 0, st, c, b->dRounds, b->dItems, b->dArgs,
                                            b->dPaths, b->ws.q[kWShadow], b->wctr.baseOf(level, kWShadow),
                                            b->wctr.countOf(level, kWShadow), b->ws, level);
-                        hipLaunchKernelGGL(k_bw_rays<2>, dim3(gclose), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
+                        hipLaunchKernelGGL(k_bw_rays<2>, dim3(gt), dim3(64), 0, st, c, b->dRounds, b->dItems, b->dArgs,
                                            b->dPaths, b->ws.q[kWBsdf], b->wctr.baseOf(level, kWBsdf),
                                            b->wctr.countOf(level, kWBsdf), b->ws, level);
                         hipLaunchKernelGGL(k_bw_finish, dim3(gfin), dim3(block), 0, st, c, b->dRounds, b->dItems, b->dArgs,
@@ -797,7 +807,7 @@ static bool enqueue_round(Batch *b, hipStream_t st) {
                 hipLaunchKernelGGL(k_batch_plan, dim3(1), dim3(64), 0, st, b->dCursor, b->dRounds, b->dItems, b->ctr,
                                    level, chunk, b->ctr.base + (size_t)level * (b->ctr.maxItems + 1), -1);
                 const bool drain = drainLevel > 0 && level >= drainLevel;
-                hipLaunchKernelGGL(drain ? kdrain : kern, dim3(grid), dim3(block), 0, st, b->dCursor, b->dRounds,
+                hipLaunchKernelGGL(drain ? kdrain : kern, dim3(grid), dim3(64), 0, st, b->dCursor, b->dRounds,
                                    b->dItems, b->dArgs, b->dPaths, b->dQ[level & 1], b->dQ[(level + 1) & 1], b->ctr,
                                    level, chunk);
                 if (drain) break;
@@ -972,15 +982,18 @@ extern "C" void *gz_batch_create(const GzBatchScene *scenes, int32_t sceneCount,
             !hip_ok(hipMalloc(&b->dQ[0], slots * sizeof(int)), "batch queue") ||
             !hip_ok(hipMalloc(&b->dQ[1], slots * sizeof(int)), "batch queue") ||
             !hip_ok(hipMalloc(&b->ctr.n, (size_t)(b->levels + 1) * b->ctr.maxItems * sizeof(unsigned)), "batch counters") ||
-            !hip_ok(hipMalloc(&b->ctr.head, (size_t)b->levels * sizeof(unsigned)), "batch counters") ||
             !hip_ok(hipMalloc(&b->ctr.base, (size_t)b->levels * (b->ctr.maxItems + 1) * sizeof(unsigned)),
                     "batch counters")) {
                 free_batch(b);
                 return nullptr;
         }
-        // Default launch: wavefront rounds when some scene is large enough for the wavefront kernels.
+        // Default launch: wavefront rounds when some scene is large enough for the wavefront kernels; rounds
+        // of few paths run whole (see launch_for for why). Eight scenes of up to 22K triangles, depth 6, levels /
+        // whole in ms: 12K paths 3.4 / 1.1, 340K 4.6 / 1.8, 1.1M 5.4 / 3.0; twelve scenes 2.9M paths 6.7 / 4.9,
+        // 14M 21 / 27.
+        b->wholePaths = b->roundPaths <= (b->anyWave ? kWholeRoundWavefront : kWholeRoundMega);
         if (b->anyWave) {
-                if (!ensure_wave(b)) {
+                if (!b->wholePaths && !ensure_wave(b)) {
                         free_batch(b);
                         return nullptr;
                 }
@@ -1064,6 +1077,7 @@ extern "C" int gz_batch_set_launch(void *batch, const GzMisLaunch *launch) {
                         return GZ_E_ALLOC;
         }
         b->launch = c;
+        b->wholePaths = false;
         release_graph(b);  // captured with the old shape
         return GZ_OK;
 }

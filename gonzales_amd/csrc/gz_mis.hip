@@ -284,9 +284,10 @@ __global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_mis_queue(MisArgs a
 template <bool kStats, int kAll>
 __global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_mis_drain(MisArgs a, GzPath *__restrict__ paths, unsigned count,
                                                                 const int *__restrict__ qin, const unsigned *nptr,
-                                                                uint32_t *__restrict__ stats) {
+                                                                unsigned perWave, uint32_t *__restrict__ stats) {
         const unsigned nin = qin ? *nptr : count;
-        for (size_t j = (size_t)blockIdx.x * 64 + threadIdx.x; j < nin; j += (size_t)gridDim.x * 64) {
+        if (threadIdx.x >= perWave) return;
+        for (size_t j = (size_t)blockIdx.x * perWave + threadIdx.x; j < nin; j += (size_t)gridDim.x * perWave) {
                 const int i = qin ? qin[j] : (int)j;
                 for (int b = 0; b <= a.maxDepth; ++b)
                         if (!bounce_one<kStats, kAll, false, 64>(a, paths, i, stats, AdjArgs{nullptr, nullptr}, nullptr)) break;
@@ -600,6 +601,13 @@ static unsigned queue_grid(Scene *s, K kern, int block, int64_t count, unsigned 
 // known to the device alone, and the waves past it only start and end).
 static unsigned rays_grid(const Scene *s, int64_t count) {
         return (unsigned)std::max<int64_t>(1, std::min<int64_t>((int64_t)s->cuCount * 256, (count + 63) / 64));
+}
+
+// 64, but 16 for up to 2^16 paths of scenes with more than the diffuse BSDF: a wave runs the union of its
+// paths' branches, and that few paths leave SIMDs idle (20K-triangle sphere, 8K paths 1.03 -> 0.93 ms, 30K
+// 1.12 -> 0.99, 120K at 16 a wave 1.39 -> 1.50; the diffuse Cornell box 8K paths 0.218 -> 0.233).
+unsigned gz::wave_paths(int64_t count, int bsdfSet) {
+        return bsdfSet != kBsdfDiffuse && count <= 1 << 16 ? 16u : 64u;
 }
 
 // Grid of k_wf_split: up to 8 blocks per CU, no more than the first level has tiles.
@@ -1133,7 +1141,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                         uint8_t *occ = keep ? rec->occ + (size_t)level * (size_t)count : q->occ;
                         if (c.drainLevel > 0 && level >= c.drainLevel) {
                                 hipLaunchKernelGGL(kdrain, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
-                                                   &lv->qn, stats);
+                                                   &lv->qn, 64u, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
                         hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin, &lv->qn,
@@ -1189,7 +1197,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                         int *qout = q->q[(level + 1) & 1];
                         if (c.drainLevel > 0 && level >= c.drainLevel) {
                                 hipLaunchKernelGGL(kdrain, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
-                                                   &q->wctl[level].qn, stats);
+                                                   &q->wctl[level].qn, 64u, stats);
                                 return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                         }
                         hipLaunchKernelGGL(ktrace, dim3(tgrid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,
@@ -1216,8 +1224,9 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 auto kdrain = d_stats ? pick_set(bset, k_mis_drain<true, 0>, k_mis_drain<true, 1>, k_mis_drain<true, 2>)
                                       : pick_set(bset, k_mis_drain<false, 0>, k_mis_drain<false, 1>, k_mis_drain<false, 2>);
                 if (lc.wholePaths) {
-                        hipLaunchKernelGGL(kdrain, dim3(rays_grid(s, count)), dim3(64), 0, st, a, d_paths, (unsigned)count,
-                                           nullptr, nullptr, stats);
+                        const unsigned per = wave_paths(count, bset);
+                        hipLaunchKernelGGL(kdrain, dim3((unsigned)((count + per - 1) / per)), dim3(64), 0, st, a, d_paths,
+                                           (unsigned)count, nullptr, nullptr, per, stats);
                         return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                 }
                 const int levels = params->maxDepth + 2;
@@ -1231,7 +1240,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                         const int *qin = level == 0 ? nullptr : q->q[level & 1];
                         if (lc.launch.drainLevel > 0 && level >= lc.launch.drainLevel) {
                                 hipLaunchKernelGGL(kdrain, dim3(rays_grid(s, count)), dim3(64), 0, st, a, d_paths,
-                                                   (unsigned)count, qin, &q->ctl[level].n, stats);
+                                                   (unsigned)count, qin, &q->ctl[level].n, 64u, stats);
                                 break;
                         }
                         hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, a, d_paths, (unsigned)count, qin,

@@ -1032,6 +1032,8 @@ bool mis_all_diffuse(const Scene *s);
 // ones (at most kDefaultMegakernelPrims primitives), which the queued megakernel serves better.
 constexpr int64_t kDefaultMegakernelPrims = 65536;
 bool default_wavefront(const Scene *s);
+// Paths per wave of a launch that runs `count` paths whole with the kernels of a BSDF set.
+unsigned wave_paths(int64_t count, int bsdfSet);
 // The BSDF set (kBsdfDiffuse, kBsdfAll or kBsdfNoLayer) a scene's megakernel-form kernels use.
 int mis_bsdf_set(const Scene *s);
 // One of three kernel instantiations by BSDF set.

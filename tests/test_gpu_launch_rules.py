@@ -50,3 +50,25 @@ def test_default_launch_equals_the_full_relaunch(gpu, diffuse, counts):
     for n, g in zip(counts, got):
         assert np.array_equal(g, ref[:n * abi.GZ_PATH.itemsize]), n
     integ.bh.free()
+
+
+def test_whole_rounds_of_a_batch_equal_its_levels(gpu):
+    """The batch's default for small rounds against an explicit level-by-level launch: the same films."""
+    from gonzales_amd.batch import BatchEntry, SceneBatch
+    from gonzales_amd.camera import DeviceFilm
+
+    pairs = [_integrator(True), _integrator(False)]
+    entries = [BatchEntry(i, c, DeviceFilm(c)) for i, c in pairs]
+    films = []
+    for launch in (None, (256, 1, 64, 3, 3), (256, 1, 64, 0, 1)):
+        batch = SceneBatch(entries, round_paths=700_001)
+        if launch:
+            batch.set_launch(*launch)
+        batch.clear_films()
+        batch.render()
+        batch.check()
+        films.append([t.clone() for e in entries for t in (e.film.light, e.film.weight, e.film.albedo, e.film.normal)])
+        batch.close()
+    for other in films[1:]:
+        assert all((a == b).all() for a, b in zip(films[0], other))
+    assert float(films[0][0].sum()) > 0 and float(films[0][4].sum()) > 0
