@@ -87,6 +87,33 @@ __device__ __forceinline__ uint32_t zs_perm(int perm, int digit) {
         return (uint32_t)(w >> (((perm & 7) << 3) + (digit << 1))) & 3u;
 }
 
+// One permuted base-4 digit of a Morton index below 2^32: the digit at bit `shift` through the permutation
+// that the hash of the higher digits picks. `mix` is zs_dim_mix(dim). In 32 bits: the index has no
+// upper half, so the 64-bit hash input folds to higher ^ mix, and the hash's last step (x ^= x >> 16)
+// leaves the top byte, the only one used, as it is.
+__device__ __forceinline__ uint32_t zs_digit32(uint32_t morton, int shift, uint32_t mix) {
+        const uint32_t at = morton >> shift;
+        uint32_t x = (at >> 2) ^ mix;
+        x ^= x >> 16;
+        x *= 0x85ebca77u;
+        x ^= x >> 13;
+        x *= 0xc2b2ae35u;
+        const uint32_t h = x >> 24;
+        const uint32_t perm = h - 24u * ((h * 171u) >> 12);  // h % 24 for h < 256
+        constexpr uint64_t w0 = zs_perm_word(0), w1 = zs_perm_word(1), w2 = zs_perm_word(2);
+        const uint32_t sel = perm & 7u;
+        const uint32_t b0 = __builtin_amdgcn_perm((uint32_t)(w0 >> 32), (uint32_t)w0, sel);
+        const uint32_t b1 = __builtin_amdgcn_perm((uint32_t)(w1 >> 32), (uint32_t)w1, sel);
+        const uint32_t b2 = __builtin_amdgcn_perm((uint32_t)(w2 >> 32), (uint32_t)w2, sel);
+        const uint32_t b = perm < 8u ? b0 : perm < 16u ? b1 : b2;  // the permutation in the low byte
+        return (b >> ((at & 3u) << 1)) & 3u;
+}
+
+__device__ __forceinline__ uint32_t zs_dim_mix(int dim) {
+        const uint64_t m = 0x55555555ull * (uint64_t)(int64_t)dim;
+        return (uint32_t)m ^ (uint32_t)(m >> 32);
+}
+
 __device__ __forceinline__ uint64_t zs_sample_index(const ZSobolParams &p, uint64_t morton, int dim) {
         uint64_t out = 0;
         const bool odd = (p.log2spp & 1) == 1;
@@ -122,6 +149,19 @@ __device__ __forceinline__ uint64_t zs_sample_index(const ZSobolParams &p, uint6
         return out;
 }
 
+__device__ __forceinline__ float zs_scale(uint32_t v) {
+        const float f = (float)v * 2.32830643653869628906e-10f;
+        const float oneMinusEps = 1.0f - 1e-6f;
+        return oneMinusEps < f ? oneMinusEps : f;
+}
+
+// zs_sobol of an index below 2^32: the upper three bytes' table entries are 0.
+__device__ __forceinline__ float zs_sobol32(uint32_t x, int dim, uint32_t seed, const uint32_t *__restrict__ table) {
+        const uint32_t *t = table + (size_t)dim * (kSobolBytes * 256);
+        const uint32_t acc = (t[x & 255u] ^ t[256 + ((x >> 8) & 255u)]) ^ (t[512 + ((x >> 16) & 255u)] ^ t[768 + (x >> 24)]);
+        return zs_scale(zs_owen(acc, seed));
+}
+
 // sobolSample: XOR of the columns of the set bits among the 52 lowest, Owen-scrambled, scaled
 // by 2^-32 (u32 -> f32 rounds to nearest even) and clamped to 1 - 1e-6. The XOR is taken a byte
 // of the index at a time from the byte table (the same XOR regrouped): seven loads that do not
@@ -132,9 +172,7 @@ __device__ __forceinline__ float zs_sobol(uint64_t index, int dim, uint32_t seed
         uint32_t acc = t[(uint32_t)x & 255u];
 #pragma unroll
         for (int k = 1; k < kSobolBytes; ++k) acc ^= t[k * 256 + ((uint32_t)(x >> (8 * k)) & 255u)];
-        const float f = (float)zs_owen(acc, seed) * 2.32830643653869628906e-10f;
-        const float oneMinusEps = 1.0f - 1e-6f;
-        return oneMinusEps < f ? oneMinusEps : f;
+        return zs_scale(zs_owen(acc, seed));
 }
 
 struct ZSobolState {
