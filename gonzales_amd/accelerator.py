@@ -112,14 +112,26 @@ class Primitives:
         return Primitives(self.kind[order], self.mesh[order], self.tri[order], self.idx[order], self.material[order])
 
 
+def _data_bytes(dtype: np.dtype) -> np.ndarray:
+    """255 for every byte of a record that belongs to a field, 0 for padding."""
+    out = np.zeros(dtype.itemsize, np.uint8)
+    for t, offset in (f[:2] for f in dtype.fields.values()):
+        out[offset:offset + t.itemsize] = _data_bytes(t) if t.names else 255
+    return out
+
+
 def take_records(a: np.ndarray, index=None) -> np.ndarray:
     """a[index] (or a copy of a) for a structured array, with the padding bytes zero: NumPy copies
     the fields of a dtype with holes and leaves the holes of the new array uninitialised."""
-    src = a if index is None else a[index]
-    out = np.zeros(len(src), a.dtype)
-    for f in a.dtype.names:
-        out[f] = src[f]
-    return out
+    a = np.ascontiguousarray(a)
+    rows = a.view(np.uint8).reshape(len(a), a.dtype.itemsize)
+    if a.dtype.itemsize % 8 == 0:  # whole words: one gather of rows in place of one of each field
+        rows = rows.view(np.uint64)
+    out = np.array(rows) if index is None else rows[index]
+    keep = _data_bytes(a.dtype).view(out.dtype)
+    for k in np.nonzero(keep != np.iinfo(keep.dtype).max)[0]:
+        out[:, k] &= keep[k]
+    return out.reshape(-1).view(a.dtype)
 
 
 def pack_prim_ids(prims: Primitives) -> np.ndarray:
@@ -352,12 +364,12 @@ def build_bounding_hierarchy_gpu(scene: Scene, prims: Primitives, max_leaf: int 
         raise abi.GzError(abi.GZ_E_INVALID, "gz_gpu_build_scene: " + abi.last_error())
     bh.handle = h
     n = len(bh.prim_ids)
-    nodes = np.zeros(max(2 * n, 1), abi.BVH2_NODE)
+    nodes = np.empty(max(int(bh.info().nodeCount), 1), abi.BVH2_NODE)
     order = np.zeros(max(n, 1), np.int32)
     count = lib.gz_gpu_export_bvh2(h, abi.ptr(nodes), len(nodes), abi.ptr(order))
     if count < 0:
         abi.check(int(count), "gz_gpu_export_bvh2")
-    bh.nodes = nodes[:count].copy()
+    bh.nodes = nodes if count == len(nodes) else nodes[:count].copy()
     bh.prim_ids = take_records(bh.prim_ids, order[:n])
     return bh
 

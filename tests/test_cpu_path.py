@@ -163,3 +163,26 @@ def test_shade_equals_oracle():
     live = paths["active"] == 1
     assert live.sum() > 1000 and (isect["hit"][live] == 1).all() and (mats[live] == 1).all()
     assert ((mats == 2) & (isect["hit"] == 1)).any()  # some rays end on the light
+
+
+def test_take_records_gathers_rows_and_clears_padding():
+    """take_records copies whole rows: every field's bytes, zeros in the holes (also those of a nested
+    record), for records of whole words and others, any index and non-contiguous input."""
+    from gonzales_amd.accelerator import take_records
+
+    g = np.random.default_rng(0)
+    for dt in (abi.PRIM_ID, abi.MATERIAL, abi.INTERSECTION, abi.BVH2_NODE):
+        a = g.integers(0, 256, 100 * dt.itemsize, dtype=np.uint8).view(dt)
+        for index in (None, g.integers(0, 100, 77), slice(3, 50), np.arange(100) % 3 == 0):
+            src = a if index is None else a[index]
+            got = take_records(a, index)
+            assert got.dtype == dt and len(got) == len(src)
+            for f in dt.names:
+                if dt[f].names:
+                    assert all(np.array_equal(got[f][h], src[f][h]) for h in dt[f].names)
+                else:
+                    assert got[f].tobytes() == src[f].tobytes()
+        assert take_records(a[::2]).tobytes() == take_records(a, np.arange(0, 100, 2)).tobytes()
+        assert len(take_records(a[:0])) == 0
+    zero = np.frombuffer(take_records(np.frombuffer(b"\xff" * 96, abi.INTERSECTION)).tobytes(), np.uint8).reshape(2, 48)
+    assert not zero[:, 25:32].any() and not zero[:, 45:].any()
