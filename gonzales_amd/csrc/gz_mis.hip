@@ -53,14 +53,12 @@ __global__ __launch_bounds__(kMisBlock) void k_mis_adjoint(MisArgs a, GzPath *__
 // The levels' counters live in device memory and are cleared by a kernel, so a whole trace is
 // a fixed sequence of launches with no host round trip (capturable in a graph).
 struct QueueLevel {
-        unsigned n;     // entries appended to this level's queue
-        unsigned head;  // entries of this level handed out to waves
+        unsigned n;  // entries appended to this level's queue
 };
 
 __global__ void k_queue_clear(QueueLevel *ctl, int levels) {
         for (int k = threadIdx.x; k < levels; k += blockDim.x) {
                 ctl[k].n = 0u;
-                ctl[k].head = 0u;
         }
 }
 
@@ -130,7 +128,7 @@ template <typename Body>
 __device__ __forceinline__ void queue_loop(unsigned count, const int *__restrict__ qin, int *__restrict__ qout,
                                            QueueLevel *ctl, int level, unsigned chunk, Body &&body) {
         const unsigned nin = qin ? ctl[level].n : count;
-        queue_run(nin, qin, &ctl[level].head, qout, &ctl[level + 1].n, chunk, body);
+        queue_run(nin, qin, nullptr, qout, &ctl[level + 1].n, chunk, body);
 }
 
 // ---- Split wavefront: one trace kernel and two shade kernels per bounce level ----------------
@@ -323,8 +321,7 @@ __global__ __launch_bounds__(kMisBlock, kAll == kBsdfAll ? 2 : 3) void k_mis_adj
 // replays its path's remaining bounces; the block flushes its LDS accumulators once at the end.
 template <int kAll>
 __global__ __launch_bounds__(kMisBlock, kAll == kBsdfAll ? 2 : 3) void k_mis_adjoint_drain(MisArgs a, GzPath *__restrict__ paths,
-                                                                 const int *__restrict__ qin, const unsigned *nptr,
-                                                                 unsigned *head, unsigned chunk, AdjArgs adj) {
+                                                                 const int *__restrict__ qin, const unsigned *nptr, AdjArgs adj) {
         __shared__ double sg[kAdjLdsMats * 4];
         const bool useLds = a.nMats <= kAdjLdsMats;
         if (useLds) {
@@ -332,18 +329,10 @@ __global__ __launch_bounds__(kMisBlock, kAll == kBsdfAll ? 2 : 3) void k_mis_adj
                 __syncthreads();
         }
         const unsigned nin = *nptr;
-        const int lane = (int)(threadIdx.x & 63);
-        for (;;) {
-                unsigned c = 0;
-                if (lane == 0) c = atomicAdd(head, chunk);
-                c = __shfl(c, 0);
-                if (c >= nin) break;
-                const unsigned end = nin - c < chunk ? nin : c + chunk;
-                for (unsigned j = c + (unsigned)lane; j < end; j += 64) {
-                        const int i = qin[j];
-                        for (int b = 0; b <= a.maxDepth; ++b)
-                                if (!bounce_one<false, kAll, true>(a, paths, i, nullptr, adj, useLds ? sg : nullptr)) break;
-                }
+        for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < nin; j += (size_t)gridDim.x * blockDim.x) {
+                const int i = qin[j];
+                for (int b = 0; b <= a.maxDepth; ++b)
+                        if (!bounce_one<false, kAll, true>(a, paths, i, nullptr, adj, useLds ? sg : nullptr)) break;
         }
         if (useLds) {
                 __syncthreads();
@@ -979,7 +968,7 @@ bool gz::mis_args(Scene *s, const GzMisParams *params, int *err, MisArgs &a) {
 template <typename K, typename Launch>
 static int queued_levels(Scene *s, MisQueues *&owner, K kern, int64_t count, int maxDepth, hipStream_t st,
                          const char *who, Launch &&launch,
-                         const std::function<void(unsigned, const int *, unsigned *, unsigned *, unsigned)> &drain = {}) {
+                         const std::function<void(unsigned, const int *, unsigned *)> &drain = {}) {
         const int levels = maxDepth + 2;
         MisQueue *q = mis_queue(owner, st, (size_t)count, levels);
         if (!q) return GZ_E_ALLOC;
@@ -992,7 +981,7 @@ static int queued_levels(Scene *s, MisQueues *&owner, K kern, int64_t count, int
                 const int *qin = level == 0 ? nullptr : q->q[level & 1];
                 int *qout = q->q[(level + 1) & 1];
                 if (drain && level >= c.drainLevel) {
-                        drain(grid, qin, &q->ctl[level].n, &q->ctl[level].head, chunk);
+                        drain(grid, qin, &q->ctl[level].n);
                         return hip_ok(hipGetLastError(), who) ? GZ_OK : GZ_E_HIP;
                 }
                 launch(level, grid, qin, qout, q->ctl, chunk);
@@ -1379,11 +1368,10 @@ static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adj
                 auto kern = pick_set(bset, k_mis_adjoint_queue<0>, k_mis_adjoint_queue<1>, k_mis_adjoint_queue<2>);
                 auto kdrain = pick_set(bset, k_mis_adjoint_drain<0>, k_mis_adjoint_drain<1>, k_mis_adjoint_drain<2>);
                 const int block = s->misLaunch.block;
-                std::function<void(unsigned, const int *, unsigned *, unsigned *, unsigned)> drain;
+                std::function<void(unsigned, const int *, unsigned *)> drain;
                 if (s->misLaunch.drainLevel > 0)
-                        drain = [&](unsigned grid, const int *qin, unsigned *n, unsigned *head, unsigned chunk) {
-                                hipLaunchKernelGGL(kdrain, dim3(grid), dim3(block), 0, st, a, d_paths, qin, n, head, chunk,
-                                                   adj);
+                        drain = [&](unsigned grid, const int *qin, unsigned *n) {
+                                hipLaunchKernelGGL(kdrain, dim3(grid), dim3(block), 0, st, a, d_paths, qin, n, adj);
                         };
                 return queued_levels(
                         s, s->misQueues, kern, count, params->maxDepth, st, "MIS adjoint launch",

@@ -47,11 +47,13 @@ class DiffRenderer:
         self.d_record = None
         self.recorded_levels = 0  # levels the last render recorded (0: none; backward traces every ray)
         if record:
-            # the full wavefront for every level (no drain), so that the record holds every level
-            # and the backward traces nothing: on the 512^2 x 32 spp inverse-rendering frame the
-            # forward takes 18.1 ms against 17.8 with the default drain from level 3, the backward
-            # 10.6 against 12.6 ms
-            self.integrator.set_launch(3, 256, 1, 64, 0)
+            # The full wavefront, recording every level it runs (the backward then traces nothing there).
+            # From 2^20 paths on every level; below, the last levels hold too few paths to fill the chip
+            # twice each, and a drain from level 2 (up to 2^18 paths) or 3 is faster for both passes although
+            # it records nothing. Step of a room with 50K triangles, depth 5, drain 0 / 2 / 3 in ms: 16K paths
+            # 1.51 / 1.34 / 1.46, 65K 2.21 / 1.88 / 2.09, 262K 2.72 / 2.27 / 2.52, 1M 4.59 / 5.46 / 4.29, 4.2M
+            # 12.9 / 17.7 / 13.3.
+            self.integrator.set_launch(3, 256, 1, 64, 2 if n <= 1 << 18 else 3 if n <= 1 << 20 else 0)
 
     def set_parameters(self, albedo=None, roughness=None) -> None:
         """albedo: (M, 3) reflectances (used where the material is diffuse); roughness: (M,)
