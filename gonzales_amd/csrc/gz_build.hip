@@ -37,7 +37,7 @@ namespace gz {
 constexpr int kBuildBlock = 256;
 
 // flags[0] bits
-enum : int { kFlagUnsafe = 1, kFlagSkip = 2, kFlagBadIndex = 4, kFlagBadTree = 8 };
+enum : int { kFlagUnsafe = 1, kFlagSkip = 2, kFlagBadIndex = 4, kFlagBadTree = 8, kFlagLoose = 16 };
 
 struct Box {
         float lo[3], hi[3];
@@ -117,6 +117,8 @@ __global__ __launch_bounds__(kBuildBlock) void k_gather(const PrimId_C *__restri
                                 c[a] = 0.5f * (b.lo[a] + b.hi[a]);
                                 // the traversal's fast slab form needs finite boxes within 2^40
                                 if (!(b.lo[a] >= -0x1p40f && b.hi[a] <= 0x1p40f)) atomicOr(&flags[0], kFlagUnsafe);
+                                // fminf and fmaxf drop a NaN: the box does not hold that vertex
+                                if (isnan(v[0][a]) || isnan(v[1][a]) || isnan(v[2][a])) atomicOr(&flags[0], kFlagLoose);
                         }
                         valid = true;
                 }
@@ -1217,8 +1219,9 @@ extern "C" void *gz_gpu_build_scene(const PrimId_C *prims, int64_t nPrims, const
                 const bool rootLeaf = sah ? h[1] == 0 : n <= maxLeaf;
                 s->nodeRecords = rootLeaf ? 0 : h[1];  // records numbered depth first, densely
                 s->triCount = n;
-                // finite boxes within 2^40, none empty; min/max of what they hold, so nested
-                s->boxes = (h[0] & (kFlagUnsafe | kFlagSkip)) ? 0 : kBoxesBounded | kBoxesNested;
+                // finite boxes within 2^40, none empty; min/max of what they hold, so nested but for NaNs
+                s->boxes = (h[0] & (kFlagUnsafe | kFlagSkip) ? 0 : kBoxesBounded) |
+                           (h[0] & (kFlagUnsafe | kFlagSkip | kFlagLoose) ? 0 : kBoxesNested);
                 if (rootLeaf) {
                         s->rootDesc = ~0;
                         s->interiorCount = 0;

@@ -8,7 +8,8 @@ triangles (the cull is then off).
 import numpy as np
 import pytest
 
-from gonzales_amd import scenes
+from gonzales_amd import abi, scenes
+from gonzales_amd.accelerator import Primitives, Scene, TriangleMesh, build_bounding_hierarchy_gpu
 from helpers import OracleView, random_rays, random_soup_hierarchy
 from test_gpu_traversal import _assert_hits_equal, _device_any, _device_closest
 
@@ -90,6 +91,35 @@ def test_boxes_that_do_not_hold_their_triangles(gpu):
     ref, _ = OracleView(bh).closest(rays, tmax)
     hits, _ = _device_closest(bh, rays, tmax)
     _assert_hits_equal(hits, ref)
+    bh.free()
+
+
+@pytest.mark.parametrize("sah", [False, True])
+@pytest.mark.parametrize("broken", [0, 1, 60])
+def test_hierarchies_built_on_the_device(gpu, sah, broken):
+    """A vertex coordinate that is NaN leaves its triangle's box finite (minima and maxima drop it) and the
+    triangle outside that box: tri_test accepts a NaN, so such a hierarchy culls nothing."""
+    n = 3000
+    g = np.random.default_rng(21)
+    v = (g.random((n, 1, 3)) + 0.1 * (g.random((n, 3, 3)) - 0.5)).astype(np.float32)
+    for k in g.permutation(n)[:broken]:
+        v[k, g.integers(0, 3), g.integers(0, 3)] = np.nan
+    mats = np.zeros(1, abi.MATERIAL)
+    mats["type"] = 1
+    scene = Scene([TriangleMesh.from_xyz(v.reshape(-1, 3), np.arange(3 * n, dtype=np.int64))], mats)
+    bh = build_bounding_hierarchy_gpu(scene, Primitives.geometric(0, n, 0), sah=sah)
+    rays, tmax = _zero_axis_rays(20_000, 22, bh)
+    for f in ("orgX", "orgY", "orgZ"):  # origins taken from a vertex may be its NaN
+        rays[f][np.isnan(rays[f])] = 0.5
+    ref, _ = OracleView(bh).closest(rays, tmax)
+    hits, _ = _device_closest(bh, rays, tmax)
+    hit = ref["hit"].astype(bool)
+    assert np.array_equal(hits["prim"] >= 0, hit)
+    assert bool(np.isnan(ref["tHit"][hit]).any()) == (broken > 0)
+    for f, r in (("t", "tHit"), ("u", "u"), ("v", "v")):
+        assert np.array_equal(hits[f][hit], ref[r][hit], equal_nan=True)
+    occ, _ = _device_any(bh, rays, tmax)
+    assert np.array_equal(occ, hit)
     bh.free()
 
 
