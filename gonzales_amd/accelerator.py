@@ -128,6 +128,8 @@ def take_records(a: np.ndarray, index=None) -> np.ndarray:
     if a.dtype.itemsize % 8 == 0:  # whole words: one gather of rows in place of one of each field
         rows = rows.view(np.uint64)
     out = np.array(rows) if index is None else rows[index]
+    if out.base is not None:  # a slice: a view of the caller's records
+        out = out.copy()
     keep = _data_bytes(a.dtype).view(out.dtype)
     for k in np.nonzero(keep != np.iinfo(keep.dtype).max)[0]:
         out[:, k] &= keep[k]

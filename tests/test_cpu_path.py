@@ -186,3 +186,18 @@ def test_take_records_gathers_rows_and_clears_padding():
         assert len(take_records(a[:0])) == 0
     zero = np.frombuffer(take_records(np.frombuffer(b"\xff" * 96, abi.INTERSECTION)).tobytes(), np.uint8).reshape(2, 48)
     assert not zero[:, 25:32].any() and not zero[:, 45:].any()
+
+
+def test_take_records_of_a_slice_is_a_copy():
+    """A slice gives records of their own: the caller's array keeps its padding bytes, read-only input is
+    taken, and writing to the result does not reach the caller's array."""
+    from gonzales_amd.accelerator import take_records
+
+    raw = bytes(range(1, 97)) * 2
+    for a in (np.frombuffer(bytearray(raw), abi.INTERSECTION), np.frombuffer(raw, abi.INTERSECTION)):
+        for index in (slice(0, 2), slice(3, None, -1), slice(None)):
+            got = take_records(a, index)
+            assert not np.shares_memory(got, a) and a.tobytes() == raw
+            assert got["tHit"].tobytes() == a[index]["tHit"].tobytes()
+            got["tHit"] = 1.0
+            assert a.tobytes() == raw
