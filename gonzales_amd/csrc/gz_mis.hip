@@ -53,12 +53,14 @@ __global__ __launch_bounds__(kMisBlock) void k_mis_adjoint(MisArgs a, GzPath *__
 // The levels' counters live in device memory and are cleared by a kernel, so a whole trace is
 // a fixed sequence of launches with no host round trip (capturable in a graph).
 struct QueueLevel {
-        unsigned n;  // entries appended to this level's queue
+        unsigned n;     // entries appended to this level's queue
+        unsigned head;  // entries handed out to waves (the replay of large frames)
 };
 
 __global__ void k_queue_clear(QueueLevel *ctl, int levels) {
         for (int k = threadIdx.x; k < levels; k += blockDim.x) {
                 ctl[k].n = 0u;
+                ctl[k].head = 0u;
         }
 }
 
@@ -121,14 +123,6 @@ __device__ __forceinline__ void queue_run(unsigned nin, const int *__restrict__ 
         int *const qo[1] = {qout};
         unsigned *const on[1] = {outN};
         queue_run_n<1>(nin, qin, head, chunk, qo, on, [&](int i) { return body(i) ? 1u : 0u; });
-}
-
-// The level form: entries of level `level` (identity at level 0), survivors to level + 1.
-template <typename Body>
-__device__ __forceinline__ void queue_loop(unsigned count, const int *__restrict__ qin, int *__restrict__ qout,
-                                           QueueLevel *ctl, int level, unsigned chunk, Body &&body) {
-        const unsigned nin = qin ? ctl[level].n : count;
-        queue_run(nin, qin, nullptr, qout, &ctl[level + 1].n, chunk, body);
 }
 
 // ---- Split wavefront: one trace kernel and two shade kernels per bounce level ----------------
@@ -293,21 +287,23 @@ __global__ __launch_bounds__(64, mis_min_waves(kAll)) void k_mis_drain(MisArgs a
 }
 
 // The replayed bounce over the same queues; a persistent block flushes its LDS gradient
-// accumulators once, when the level is drained.
+// accumulators once, when the level is drained. `shared`: waves take their entries from the level's one
+// counter instead of by striding (replay_shares_head).
 template <int kAll>
 __global__ __launch_bounds__(kMisBlock, kAll == kBsdfAll ? 2 : 3) void k_mis_adjoint_queue(MisArgs a, GzPath *__restrict__ paths,
                                                                  unsigned count, const int *__restrict__ qin,
                                                                  int *__restrict__ qout, QueueLevel *ctl, int level,
-                                                                 unsigned chunk, AdjArgs adj) {
+                                                                 unsigned chunk, AdjArgs adj, bool shared) {
         __shared__ double sg[kAdjLdsMats * 4];
         const bool useLds = a.nMats <= kAdjLdsMats;
         if (useLds) {
                 for (int k = threadIdx.x; k < a.nMats * 4; k += blockDim.x) sg[k] = 0.0;
                 __syncthreads();
         }
-        queue_loop(count, qin, qout, ctl, level, chunk, [&](int i) {
-                return bounce_one<false, kAll, true>(a, paths, i, nullptr, adj, useLds ? sg : nullptr);
-        });
+        queue_run(qin ? ctl[level].n : count, qin, shared ? &ctl[level].head : nullptr, qout, &ctl[level + 1].n, chunk,
+                  [&](int i) {
+                          return bounce_one<false, kAll, true>(a, paths, i, nullptr, adj, useLds ? sg : nullptr);
+                  });
         if (useLds) {
                 __syncthreads();
                 for (int k = threadIdx.x; k < a.nMats * 4; k += blockDim.x) {
@@ -1328,6 +1324,12 @@ extern "C" int gz_gpu_mis_trace_stats_device(void *handle, GzPath *d_paths, int6
         return mis_launch(handle, d_paths, count, params, d_stats, stream, true, "gz_gpu_mis_trace_stats_device");
 }
 
+// Whether a replay of `count` paths hands its queue entries out through one counter a level. Striding has no
+// counter that all waves hit, but leaves the waves with the longest paths to finish alone. Room with 50K
+// triangles, depth 5, strided / shared in ms, from the record: 262K paths 1.07 / 1.14, 1.3M 1.71 / 1.88, 2.1M
+// 2.12 / 2.09, 4.2M 5.6 / 5.1, 8.4M 10.7 / 9.5; tracing its rays again: 2.1M 3.6 / 3.2, 8.4M 17.9 / 15.5.
+static bool replay_shares_head(int64_t count) { return count > (int64_t)3 << 19; }
+
 // The adjoint replay; rec: the forward pass's replay record (null: every ray is traced again).
 static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adjoint, int64_t count,
                        const GzMisParams *params, double *d_grad, void *stream, const MisRecord *rec) {
@@ -1368,6 +1370,7 @@ static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adj
                 auto kern = pick_set(bset, k_mis_adjoint_queue<0>, k_mis_adjoint_queue<1>, k_mis_adjoint_queue<2>);
                 auto kdrain = pick_set(bset, k_mis_adjoint_drain<0>, k_mis_adjoint_drain<1>, k_mis_adjoint_drain<2>);
                 const int block = s->misLaunch.block;
+                const bool shared = replay_shares_head(count);
                 std::function<void(unsigned, const int *, unsigned *)> drain;
                 if (s->misLaunch.drainLevel > 0)
                         drain = [&](unsigned grid, const int *qin, unsigned *n) {
@@ -1377,7 +1380,7 @@ static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adj
                         s, s->misQueues, kern, count, params->maxDepth, st, "MIS adjoint launch",
                         [&](int level, unsigned grid, const int *qin, int *qout, QueueLevel *ctl, unsigned chunk) {
                                 hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, a, d_paths, (unsigned)count, qin,
-                                                   qout, ctl, level, chunk, adj);
+                                                   qout, ctl, level, chunk, adj, shared);
                         },
                         drain);
         }

@@ -72,3 +72,35 @@ def test_whole_rounds_of_a_batch_equal_its_levels(gpu):
     for other in films[1:]:
         assert all((a == b).all() for a, b in zip(films[0], other))
     assert float(films[0][0].sum()) > 0 and float(films[0][4].sum()) > 0
+
+
+@pytest.mark.parametrize("res,spp", [((512, 384), 8), ((512, 385), 8)])
+def test_replay_of_large_frames_equals_the_full_relaunch(gpu, res, spp):
+    """The queued replay on both sides of 3 x 2^19 paths (strided below and at it, one shared counter a level
+    above), from a record and tracing its rays again, against one launch per bounce over all paths: the same
+    path records and gradients. The gradients are float64 sums of up to 1e7 terms of one sign (the target is
+    black) in another order: 1e7 x 2^-53 = 1.1e-9 of the largest, times four for the terms of the other sign."""
+    import torch
+    from gonzales_amd.camera import Film, PerspectiveCamera, pbrt_transform
+    from gonzales_amd.diff import DiffRenderer
+
+    bh, gz, _, _ = scenes.inverse_rendering_scene(subdivisions=3, n_params=8)
+    bh.upload_to_gpu()
+    cam = PerspectiveCamera(pbrt_transform([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, -1, 0, 0, -1, 6.8, 1]), 19.5, Film(*res), spp, 0)
+    assert cam.path_count == res[0] * res[1] * spp
+    opt = MisOptions(max_depth=3, zsobol_seed=cam.c.zsSeed, log2_spp=cam.c.zsLog2Spp, base4_digits=cam.c.zsBase4Digits)
+    r = DiffRenderer(bh, cam, gz, opt)
+    out = []
+    for launch, record in (((0, 256, 1, 256, 0), False), ((3, 256, 1, 64, 0), True), ((3, 256, 1, 64, 2), True),
+                           ((1, 128, 1, 256, 0), False)):
+        r.integrator.set_launch(*launch)
+        img = r.render()
+        assert (r.recorded_levels > 0) == record
+        ga, gr = r.backward(2 * img)
+        out.append((ga, gr, r.d_paths.clone()))
+    for ga, gr, paths in out[1:]:
+        assert torch.equal(paths, out[0][2])
+        for x, y in ((ga, out[0][0]), (gr, out[0][1])):
+            assert float(y.abs().max()) > 0
+            assert float((x - y).abs().max()) <= 5e-9 * float(y.abs().max())
+    bh.free()
