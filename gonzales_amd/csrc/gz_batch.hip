@@ -699,9 +699,28 @@ static bool upload(T **dst, const T *src, size_t count, const char *what) {
         return count == 0 || hip_ok(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice), what);
 }
 
-// Rounds of at most this many paths run whole under the default launch (with and without scenes that
-// default to the wavefront).
-constexpr int64_t kWholeRoundWavefront = 3 << 20, kWholeRoundMega = 1 << 19;
+// Under the default launch a round runs whole (see launch_for for why) if it has at most kWholeRoundWave paths
+// of scenes that default to the wavefront and kWholeRoundPaths in all, or, without such a scene, at most
+// kWholeRoundMega. Wavefront levels / whole in ms, depth 8, wavefront scenes alone: twelve 20K-triangle spheres
+// that fill their frames 0.74M paths 4.5 / 4.5, 1.03M 4.9 / 5.6, 1.23M 5.0 / 6.6, 3.1M 9.2 / 14.2; one of 300K
+// triangles 0.74M 5.6 / 5.0, 1.05M 7.0 / 6.8, 2.9M 9.9 / 14.2. With small diffuse scenes beside them the whole
+// paths' limit is the wavefront scenes' part: eleven Cornell boxes and a sphere 3.1M (0.26M) 8.7 / 6.1, twelve
+// mixed scenes 1.5M (1.0M) 5.1 / 4.0.
+constexpr int64_t kWholeRoundWave = 1 << 20, kWholeRoundPaths = 3 << 20, kWholeRoundMega = 1 << 19;
+
+static bool whole_rounds(const Batch *b) {
+        int64_t most = 0;  // paths of wavefront scenes in a round
+        for (const BatchRound &r : b->hRounds) {
+                int64_t n = 0;
+                for (int k = 0; k < r.nItems; ++k) {
+                        const BatchItem &it = b->hItems[(size_t)(r.firstItem + k)];
+                        if (it.wave) n += it.count;
+                }
+                most = std::max(most, n);
+        }
+        if (!b->anyWave) return b->roundPaths <= kWholeRoundMega;
+        return most <= kWholeRoundWave && b->roundPaths <= kWholeRoundPaths;
+}
 
 // Enqueues one round's launch sequence on `st`.
 static bool enqueue_round(Batch *b, hipStream_t st) {
@@ -988,10 +1007,8 @@ extern "C" void *gz_batch_create(const GzBatchScene *scenes, int32_t sceneCount,
                 return nullptr;
         }
         // Default launch: wavefront rounds when some scene is large enough for the wavefront kernels; rounds
-        // of few paths run whole (see launch_for for why). Eight scenes of up to 22K triangles, depth 6, levels /
-        // whole in ms: 12K paths 3.4 / 1.1, 340K 4.6 / 1.8, 1.1M 5.4 / 3.0; twelve scenes 2.9M paths 6.7 / 4.9,
-        // 14M 21 / 27.
-        b->wholePaths = b->roundPaths <= (b->anyWave ? kWholeRoundWavefront : kWholeRoundMega);
+        // of few paths run whole.
+        b->wholePaths = whole_rounds(b);
         if (b->anyWave) {
                 if (!b->wholePaths && !ensure_wave(b)) {
                         free_batch(b);

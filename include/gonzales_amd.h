@@ -616,8 +616,9 @@ int gz_batch_info(void *batch, struct GzBatchInfo *info);
 /* Launch shape of the batch's bounce levels (queued 1 or 3, as in GzMisLaunch). queued 3 bounces
  * the items of the scenes whose own default launch is the wavefront with the wavefront kernels and
  * the others with the bounce kernel, level by level. The default is {3, 256, 1, 64, 3} when some
- * scene's default is the wavefront, else {1, 256, 1, 256, 3}; until one is set, rounds of up to 3 x 2^20
- * paths (2^19 without a wavefront scene) run each path whole, in one launch. */
+ * scene's default is the wavefront, else {1, 256, 1, 256, 3}; until one is set, batches
+ * whose rounds hold at most 2^20 paths of wavefront scenes and 3 x 2^20 in all (2^19 without a wavefront
+ * scene) run each path whole, in one launch. */
 int gz_batch_set_launch(void *batch, const struct GzMisLaunch *launch);
 /* Renders every path of every scene once and adds it to the scenes' films, asynchronously on
  * `stream`. Each round is the same launch sequence (camera rays, device path queues per bounce

@@ -74,6 +74,30 @@ def test_whole_rounds_of_a_batch_equal_its_levels(gpu):
     assert float(films[0][0].sum()) > 0 and float(films[0][4].sum()) > 0
 
 
+def test_rounds_on_both_sides_of_the_wavefront_scenes_line(gpu):
+    """Default rounds with 2^20 and with 2^20 + 8 paths of a scene that defaults to the wavefront (whole paths
+    and levels): the films of an explicit level-by-level launch."""
+    from gonzales_amd.batch import BatchEntry, SceneBatch
+    from gonzales_amd.camera import DeviceFilm
+
+    (mixed, cam), (diffuse, dcam) = _integrator(False), _integrator(True)
+    entries = [BatchEntry(mixed, cam, DeviceFilm(cam)), BatchEntry(diffuse, dcam, DeviceFilm(dcam))]
+    films = []
+    for round_paths, launch in ((1 << 20, None), ((1 << 20) + 8, None), (1 << 20, (256, 1, 64, 0, 1))):
+        batch = SceneBatch(entries, round_paths=round_paths)
+        if launch:
+            batch.set_launch(*launch)
+        for use_graph in (True, False):
+            batch.clear_films()
+            batch.render(use_graph)
+            batch.check()
+            films.append([t.clone() for e in entries for t in (e.film.light, e.film.weight, e.film.albedo, e.film.normal)])
+        batch.close()
+    for other in films[1:]:
+        assert all((a == b).all() for a, b in zip(films[0], other))
+    assert float(films[0][0].sum()) > 0 and float(films[0][4].sum()) > 0
+
+
 @pytest.mark.parametrize("res,spp", [((512, 384), 8), ((512, 385), 8)])
 def test_replay_of_large_frames_equals_the_full_relaunch(gpu, res, spp):
     """The queued replay on both sides of 3 x 2^19 paths (strided below and at it, one shared counter a level
