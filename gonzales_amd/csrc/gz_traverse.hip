@@ -485,7 +485,7 @@ __global__ __launch_bounds__(kBlock) void k_expand(const GzHit *__restrict__ hit
 
 static inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-// Whether a batch is traced by k_trace with its rays in the given order: while the caller has set no
+// Whether a batch is traced by k_trace (in the given order but for bin_plain): while the caller has set no
 // launch configuration, below kPersistentMinRays rays. Persistent lanes keep more of a wave busy on long
 // incoherent rays, but refilling them from a wave's own reserve leaves a tail that only a large batch
 // hides, and binning costs two passes over the rays. A million-triangle soup, incoherent rays, k_trace /
@@ -494,6 +494,17 @@ static inline unsigned grid_for(int64_t n) { return (unsigned)((n + kBlock - 1) 
 // around 50K triangles 0.35 / 1.1.
 static constexpr int64_t kPersistentMinRays = 1 << 22;
 static bool trace_plain(const Scene *s, int64_t n) { return !s->traceConfigSet && n < kPersistentMinRays; }
+
+// Whether such a batch is binned all the same: large ones on trees that the L2s do not hold. In the given
+// order incoherent rays miss them more than the binning costs, and took longer than binned persistent lanes;
+// short rays pay for it. k_trace in the given order / binned, persistent lanes binned, in ms. Soups of 400K
+// triangles 3M rays 2.8 / 2.7, 2.8, 4.2M 3.85 / 3.68, 3.5; 1M triangles 2.1M 2.70 / 2.53, 2.6, 3M 3.70 / 3.52,
+// 3.4, 4.2M 5.05 / 4.74, 4.3; 3M triangles 2.1M 3.27 / 2.95, 3.0, 4.2M 6.0 / 5.3, 4.9; 200K triangles 4.2M
+// 3.0 / 2.9, 2.9. Spheres of 1M triangles 3M 0.94 / 1.06, 1.74, 4.2M 1.15 / 1.26, 1.92; 4M triangles 2.1M
+// 0.93 / 1.05, 1.68, 4.2M 1.43 / 1.52, 2.0.
+static bool bin_plain(const Scene *s, int64_t n) {
+        return n >= (s->primCount > 1 << 21 ? (int64_t)1 << 21 : (int64_t)3 << 20) && s->primCount > 1 << 18;
+}
 
 // Rays per wave of k_trace: 64, or 32 or 16 where that still makes at most 4096 waves (4 per SIMD). A
 // batch that small leaves SIMDs idle, and a wave's step is shorter with fewer lanes loading (200,000
@@ -610,7 +621,8 @@ static const SortedRay *bin_rays(Scene *s, StreamSlot *slot, const Ray_C *d_rays
                                  hipStream_t stream, bool &failed) {
         failed = false;
         const int32_t minRays = s->traceConfig.binMinRays;
-        if (minRays <= 0 || n < minRays || trace_plain(s, n) || s->empty || s->rootDesc < 0 || n > 0xffffffffLL) return nullptr;
+        if (minRays <= 0 || n < minRays || (trace_plain(s, n) && !bin_plain(s, n))) return nullptr;
+        if (s->empty || s->rootDesc < 0 || n > 0xffffffffLL) return nullptr;
         uint32_t nBlocks, tiles;
         int64_t entries;
         const uint32_t per = bin_per(n);

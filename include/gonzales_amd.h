@@ -283,7 +283,8 @@ int gz_gpu_expand_hits_device(void *handle, const struct GzHit *d_hits, const fl
  *                 the given order;
  *   recordTimes : 1 = record HIP events around the binning and the traversal kernel of each
  *                 launch, for gz_gpu_trace_times (0 = none).
- * Until a configuration is set, batches below 2^22 rays run in mode 0 in the given order. */
+ * Until a configuration is set, batches below 2^22 rays run in mode 0, in the given order but for scenes of
+ * more than 2^18 primitives from 3 x 2^20 rays on (more than 2^21 primitives: from 2^21 rays on). */
 struct GzTraceConfig {
         int32_t persistent;
         int32_t ldsStack;

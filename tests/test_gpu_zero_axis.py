@@ -146,3 +146,22 @@ def test_default_rule_on_both_sides_of_its_line(gpu):
     sel = slice(0, 50_000)
     _assert_hits_equal(whole[sel], OracleView(bh).closest(rays[sel], tmax[sel])[0])
     bh.free()
+
+
+@pytest.mark.parametrize("n_tris,binned", [(1 << 18, False), ((1 << 18) + 1, True)])
+def test_large_default_batches_on_large_trees_are_binned(gpu, n_tris, binned):
+    """Default batches of one lane per ray: on trees of more than 2^18 primitives binned from 3 x 2^20 rays on
+    (the handle then keeps the binning's storage), with the hits of the given order."""
+    bh = random_soup_hierarchy(n_tris, 13, scale=0.01)
+    bh.upload_to_gpu()
+    rays, tmax = random_rays(3 << 20, 14)
+    part, _ = _device_closest(bh, rays[:-1], tmax[:-1])
+    before = bh.info().deviceBytes
+    whole, _ = _device_closest(bh, rays, tmax)
+    assert (bh.info().deviceBytes > before) == binned
+    assert whole[:-1].tobytes() == part.tobytes()
+    occ, _ = _device_any(bh, rays, tmax)
+    assert np.array_equal(occ, whole["prim"] >= 0)
+    sel = slice(len(rays) - 50_000, None)
+    _assert_hits_equal(whole[sel], OracleView(bh).closest(rays[sel], tmax[sel])[0])
+    bh.free()
