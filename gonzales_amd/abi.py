@@ -88,6 +88,9 @@ class GzSceneInfo(ctypes.Structure):
                 ("deviceBytes", ctypes.c_int64), ("maxDepth", ctypes.c_int32), ("rootIsLeaf", ctypes.c_int32)]
 
 
+GZ_LAUNCH_BY_SIZE = 1  # GzTraceConfig.reserved, GzMisLaunch.reserved[0]: the launch goes by the size of the work
+
+
 class GzTraceConfig(ctypes.Structure):
     _fields_ = [("persistent", ctypes.c_int32), ("ldsStack", ctypes.c_int32), ("refillLanes", ctypes.c_int32),
                 ("gridScale", ctypes.c_int32), ("chunk", ctypes.c_int32), ("binMinRays", ctypes.c_int32),

@@ -304,8 +304,11 @@ class BoundingHierarchy:
 
     def set_trace_config(self, persistent: int = 3, lds_stack: int = 16, refill_lanes: int = 32,
                          grid_scale: int = 1, chunk: int = 128, bin_min_rays: int = 1 << 18,
-                         record_times: int = 0) -> None:
-        cfg = abi.GzTraceConfig(persistent, lds_stack, refill_lanes, grid_scale, chunk, bin_min_rays, record_times)
+                         record_times: int = 0, by_size: int = 0) -> None:
+        """Launch configuration of the traversal kernels. by_size = 1 with the other defaults goes back to the
+        choice by batch size that holds until a configuration is set."""
+        cfg = abi.GzTraceConfig(persistent, lds_stack, refill_lanes, grid_scale, chunk, bin_min_rays, record_times,
+                                by_size)
         abi.check(abi.load().gz_gpu_set_trace_config(self.handle, ctypes.byref(cfg)), "gz_gpu_set_trace_config")
 
     def trace_times(self, stream=None) -> tuple[float, float]:
@@ -316,6 +319,8 @@ class BoundingHierarchy:
         return b.value, t.value
 
     def trace_config(self) -> abi.GzTraceConfig:
+        """The configuration in use (reserved = abi.GZ_LAUNCH_BY_SIZE while none is set); its fields in order
+        are set_trace_config's arguments."""
         cfg = abi.GzTraceConfig()
         abi.check(abi.load().gz_gpu_get_trace_config(self.handle, ctypes.byref(cfg)), "gz_gpu_get_trace_config")
         return cfg

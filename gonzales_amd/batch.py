@@ -60,12 +60,13 @@ class SceneBatch:
         return out
 
     def set_launch(self, block: int = 256, grid_scale: int = 1, chunk: int = 256, drain_level: int = 3,
-                   queued: int = 1) -> None:
-        """Launch shape of the batch's bounce levels: queued 1 = one persistent bounce kernel per
+                   queued: int = 1, by_size: int = 0) -> None:
+        """Launch shape of the batch's bounce levels: queued 1 = one bounce kernel per
         level, 3 = the full wavefront per level (closest hits sorted by BSDF class, shade kernels,
         shadow and BSDF rays traced by their own kernels, finish kernels); drain_level > 0 runs
-        the bounce levels from that one on in a single launch (a lane per path)."""
-        c = abi.GzMisLaunch(queued, block, grid_scale, chunk, drain_level)
+        the bounce levels from that one on in a single launch (a lane per path). by_size = 1 with the
+        other defaults goes back to the choice by scenes and round size that holds until one is set."""
+        c = abi.GzMisLaunch(queued, block, grid_scale, chunk, drain_level, (by_size, 0, 0))
         abi.check(abi.load().gz_batch_set_launch(self.handle, ctypes.byref(c)), "gz_batch_set_launch")
 
     def clear_films(self) -> None:

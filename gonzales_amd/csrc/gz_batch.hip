@@ -577,7 +577,7 @@ struct Batch {
         int maxItems = 0;
         std::vector<BatchRound> hRounds;
         std::vector<BatchItem> hItems;
-        GzMisLaunch launch{1, 256, 1, 256, 3, {0, 0, 0}};
+        GzMisLaunch launch = kMegakernelLaunch;
         bool wholePaths = false;  // a round is one launch, a lane per path through all its bounces
         int cuCount = 256;
 
@@ -720,6 +720,16 @@ static bool whole_rounds(const Batch *b) {
         }
         if (!b->anyWave) return b->roundPaths <= kWholeRoundMega;
         return most <= kWholeRoundWave && b->roundPaths <= kWholeRoundPaths;
+}
+
+// The launch until one is set: wavefront rounds when some scene defaults to the wavefront; rounds of few paths
+// run whole.
+static bool default_launch(Batch *b) {
+        const bool whole = whole_rounds(b);
+        if (b->anyWave && !whole && !ensure_wave(b)) return false;
+        b->launch = b->anyWave ? kWavefrontLaunch : kMegakernelLaunch;
+        b->wholePaths = whole;
+        return true;
 }
 
 // Enqueues one round's launch sequence on `st`.
@@ -1006,15 +1016,9 @@ extern "C" void *gz_batch_create(const GzBatchScene *scenes, int32_t sceneCount,
                 free_batch(b);
                 return nullptr;
         }
-        // Default launch: wavefront rounds when some scene is large enough for the wavefront kernels; rounds
-        // of few paths run whole.
-        b->wholePaths = whole_rounds(b);
-        if (b->anyWave) {
-                if (!b->wholePaths && !ensure_wave(b)) {
-                        free_batch(b);
-                        return nullptr;
-                }
-                b->launch = GzMisLaunch{3, 256, 1, 64, 3, {0, 0, 0}};
+        if (!default_launch(b)) {
+                free_batch(b);
+                return nullptr;
         }
         // Lanes of the scenes that render alone: each scene to the lane with the fewest paths so
         // far (lane 0 starts with the rounds' paths, which it runs first; ties to the lower lane),
@@ -1080,21 +1084,27 @@ extern "C" int gz_batch_set_launch(void *batch, const GzMisLaunch *launch) {
         const GzMisLaunch &c = *launch;
         if ((c.queued != 1 && c.queued != 3) || (c.block != 64 && c.block != 128 && c.block != 256) || c.gridScale < 1 ||
             c.gridScale > 16 || c.chunk < 64 || c.chunk > 4096 || c.chunk % 64 != 0 || c.drainLevel < 0 ||
-            c.drainLevel > 64 || c.reserved[0] != 0 || c.reserved[1] != 0 || c.reserved[2] != 0) {
+            c.drainLevel > 64 || (c.reserved[0] != 0 && c.reserved[0] != GZ_LAUNCH_BY_SIZE) || c.reserved[1] != 0 ||
+            c.reserved[2] != 0) {
                 set_error("gz_batch_set_launch: queued %d block %d gridScale %d chunk %d drainLevel %d out of range "
                           "(queued must be 1 or 3)",
                           c.queued, c.block, c.gridScale, c.chunk, c.drainLevel);
                 return GZ_E_INVALID;
         }
         Batch *b = static_cast<Batch *>(batch);
-        if (c.queued == 3) {
+        const bool bySize = launch_by_size(c);
+        if (c.queued == 3 || bySize) {
                 int cur = -1;
                 if (!hip_ok(hipGetDevice(&cur), "get device") ||
-                    (cur != b->device && !hip_ok(hipSetDevice(b->device), "set device")) || !ensure_wave(b))
+                    (cur != b->device && !hip_ok(hipSetDevice(b->device), "set device")) ||
+                    !(bySize ? default_launch(b) : ensure_wave(b)))
                         return GZ_E_ALLOC;
         }
-        b->launch = c;
-        b->wholePaths = false;
+        if (!bySize) {
+                b->launch = c;
+                b->launch.reserved[0] = 0;
+                b->wholePaths = false;
+        }
         release_graph(b);  // captured with the old shape
         return GZ_OK;
 }

@@ -89,14 +89,28 @@ struct StreamSlot {
         bool timed = false;
 };
 
+// The launches of a handle (and a batch) that none has been set for.
+constexpr GzTraceConfig kDefaultTraceConfig{3, 16, 32, 1, 128, 1 << 18, 0, 0};
+constexpr GzMisLaunch kMegakernelLaunch{1, 256, 1, 256, 3, {0, 0, 0}};
+constexpr GzMisLaunch kWavefrontLaunch{3, 256, 1, 64, 3, {0, 0, 0}};
+
+// Whether c is one of the default launches marked as the choice by size.
+inline bool launch_by_size(const GzMisLaunch &c) {
+        auto is = [&](const GzMisLaunch &d) {
+                return c.queued == d.queued && c.block == d.block && c.gridScale == d.gridScale && c.chunk == d.chunk &&
+                       c.drainLevel == d.drainLevel;
+        };
+        return c.reserved[0] == GZ_LAUNCH_BY_SIZE && (is(kMegakernelLaunch) || is(kWavefrontLaunch));
+}
+
 struct Scene {
         std::mutex mu;
         std::map<hipStream_t, StreamSlot> slots;
         uint64_t misGeneration = 0;  // bumped by every gz_gpu_set_mis_scene (batches check it)
         MisScene *mis = nullptr;
         MisQueues *misQueues = nullptr;
-        GzMisLaunch misLaunch{1, 256, 1, 256, 3, {0, 0, 0}};
-        bool misLaunchSet = false;  // false: misLaunch follows the scene (default_mis_launch)
+        GzMisLaunch misLaunch = kMegakernelLaunch;
+        bool misLaunchSet = false;  // false: misLaunch follows the scene (default_wavefront)
         int device = 0;
         hipStream_t stream = nullptr;  // used by the synchronous host-buffer entry points
 
@@ -128,8 +142,8 @@ struct Scene {
         size_t stageBytes = 0;
 
         // Traversal launch configuration.
-        GzTraceConfig traceConfig{3, 16, 32, 1, 128, 1 << 18, 0, 0};
-        bool traceConfigSet = false;  // false: smaller batches take a lane per ray, unbinned (trace_plain)
+        GzTraceConfig traceConfig = kDefaultTraceConfig;
+        bool traceConfigSet = false;  // false: smaller batches take a lane per ray (trace_plain)
         int boxes = 0;  // what is known of the node boxes: kBoxesBounded | kBoxesNested
         int cuCount = 256;
 };

@@ -998,8 +998,7 @@ bool gz::default_wavefront(const Scene *s) {
 
 static void refresh_default_launch(Scene *s) {
         if (s->misLaunchSet) return;
-        s->misLaunch = default_wavefront(s) ? GzMisLaunch{3, 256, 1, 64, 3, {0, 0, 0}}
-                                            : GzMisLaunch{1, 256, 1, 256, 3, {0, 0, 0}};
+        s->misLaunch = default_wavefront(s) ? kWavefrontLaunch : kMegakernelLaunch;
 }
 
 // The launch a trace of `count` paths takes: the handle's, once gz_gpu_set_mis_launch has set one; else the
@@ -1245,26 +1244,31 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
         return GZ_OK;
 }
 
+// Whether a launch's values are in range; says who asks if not.
+static bool launch_ok(const GzMisLaunch &c, const char *who) {
+        if (c.queued >= 0 && c.queued <= 3 && (c.block == 64 || c.block == 128 || c.block == 256) && c.gridScale >= 1 &&
+            c.gridScale <= 16 && c.chunk >= 64 && c.chunk <= 4096 && c.chunk % 64 == 0 && c.drainLevel >= 0 &&
+            c.drainLevel <= 64 && (c.queued != 0 || c.drainLevel == 0) &&
+            (c.reserved[0] == 0 || c.reserved[0] == GZ_LAUNCH_BY_SIZE) && c.reserved[1] == 0 && c.reserved[2] == 0)
+                return true;
+        set_error("%s: queued %d block %d gridScale %d chunk %d drainLevel %d out of range "
+                  "(drainLevel needs a queued mode; reserved must be zero)",
+                  who, c.queued, c.block, c.gridScale, c.chunk, c.drainLevel);
+        return false;
+}
+
 extern "C" int gz_gpu_set_mis_launch(void *handle, const GzMisLaunch *launch) {
         clear_error();
         if (!handle || !launch) {
                 set_error("gz_gpu_set_mis_launch: bad arguments");
                 return GZ_E_INVALID;
         }
-        const GzMisLaunch &c = *launch;
-        if (c.queued < 0 || c.queued > 3 || (c.block != 64 && c.block != 128 && c.block != 256) ||
-            c.gridScale < 1 || c.gridScale > 16 || c.chunk < 64 || c.chunk > 4096 || c.chunk % 64 != 0 ||
-            c.drainLevel < 0 || c.drainLevel > 64 || (c.queued == 0 && c.drainLevel != 0) || c.reserved[0] != 0 ||
-            c.reserved[1] != 0 || c.reserved[2] != 0) {
-                set_error("gz_gpu_set_mis_launch: queued %d block %d gridScale %d chunk %d drainLevel %d out of range "
-                          "(drainLevel needs a queued mode; reserved must be zero)",
-                          c.queued, c.block, c.gridScale, c.chunk, c.drainLevel);
-                return GZ_E_INVALID;
-        }
+        if (!launch_ok(*launch, "gz_gpu_set_mis_launch")) return GZ_E_INVALID;
         Scene *s = static_cast<Scene *>(handle);
         std::lock_guard<std::mutex> lock(s->mu);
-        s->misLaunch = c;
-        s->misLaunchSet = true;
+        s->misLaunchSet = !launch_by_size(*launch);
+        s->misLaunch = *launch;
+        s->misLaunch.reserved[0] = 0;
         return GZ_OK;
 }
 
@@ -1278,6 +1282,7 @@ extern "C" int gz_gpu_get_mis_launch(void *handle, GzMisLaunch *launch) {
         std::lock_guard<std::mutex> lock(s->mu);
         refresh_default_launch(s);
         *launch = s->misLaunch;
+        if (!s->misLaunchSet) launch->reserved[0] = GZ_LAUNCH_BY_SIZE;
         return GZ_OK;
 }
 

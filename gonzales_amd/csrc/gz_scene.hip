@@ -488,8 +488,13 @@ extern "C" int gz_gpu_set_trace_config(void *handle, const GzTraceConfig *config
         }
         Scene *s = static_cast<Scene *>(handle);
         std::lock_guard<std::mutex> lock(s->mu);
+        // the defaults marked as the choice by size, as get returns them while none is set: none is set
+        GzTraceConfig dflt = kDefaultTraceConfig;
+        dflt.recordTimes = config->recordTimes;
+        dflt.reserved = GZ_LAUNCH_BY_SIZE;
+        s->traceConfigSet = std::memcmp(config, &dflt, sizeof dflt) != 0;
         s->traceConfig = *config;
-        s->traceConfigSet = true;
+        if (config->reserved == GZ_LAUNCH_BY_SIZE) s->traceConfig.reserved = 0;
         return GZ_OK;
 }
 
@@ -502,5 +507,6 @@ extern "C" int gz_gpu_get_trace_config(void *handle, GzTraceConfig *config) {
         Scene *s = static_cast<Scene *>(handle);
         std::lock_guard<std::mutex> lock(s->mu);
         *config = s->traceConfig;
+        if (!s->traceConfigSet) config->reserved = GZ_LAUNCH_BY_SIZE;
         return GZ_OK;
 }

@@ -176,17 +176,30 @@ class VolumePathIntegrator:
                   "gz_gpu_mis_bounce_device")
 
     def set_launch(self, queued: int = 1, block: int = 256, grid_scale: int = 1, chunk: int = 256,
-                   drain_level: int = 0) -> None:
+                   drain_level: int = 0, by_size: int = 0) -> None:
         """Launch configuration of trace/trace_stats and the adjoint on this scene handle (the
-        results never depend on it)."""
-        c = abi.GzMisLaunch(queued, block, grid_scale, chunk, drain_level)
+        results never depend on it). by_size = 1: see reset_launch."""
+        c = abi.GzMisLaunch(queued, block, grid_scale, chunk, drain_level, (by_size, 0, 0))
         abi.check(abi.load().gz_gpu_set_mis_launch(self.bh.handle, ctypes.byref(c)), "gz_gpu_set_mis_launch")
 
+    def reset_launch(self) -> None:
+        """Back to the default launch, chosen by scene and path count, that holds until one is set."""
+        self.set_launch(1, 256, 1, 256, 3, by_size=1)
+
     def launch(self) -> tuple[int, int, int, int, int]:
-        """(queued, block, grid_scale, chunk, drain_level) of this scene handle."""
+        """(queued, block, grid_scale, chunk, drain_level) of this scene handle; of its default while
+        launch_by_size()."""
+        c = self._launch()
+        return c.queued, c.block, c.gridScale, c.chunk, c.drainLevel
+
+    def launch_by_size(self) -> bool:
+        """Whether the launch is the default (none set): chosen by scene and path count."""
+        return self._launch().reserved[0] == abi.GZ_LAUNCH_BY_SIZE
+
+    def _launch(self) -> abi.GzMisLaunch:
         c = abi.GzMisLaunch()
         abi.check(abi.load().gz_gpu_get_mis_launch(self.bh.handle, ctypes.byref(c)), "gz_gpu_get_mis_launch")
-        return c.queued, c.block, c.gridScale, c.chunk, c.drainLevel
+        return c
 
     def release_queues(self) -> None:
         """Frees the path-queue storage kept on this scene handle for its largest launch; the

@@ -263,6 +263,10 @@ int gz_gpu_traverse_any_stats_device(void *handle, const struct Ray_C *d_rays, c
 int gz_gpu_expand_hits_device(void *handle, const struct GzHit *d_hits, const float *d_tMax,
                               int64_t count, struct Intersection_C *d_results, void *stream);
 
+/* GzTraceConfig.reserved and GzMisLaunch.reserved[0] of a launch that is chosen by the size of the
+ * work, as it is until one is set. */
+#define GZ_LAUNCH_BY_SIZE 1
+
 /* Launch configuration of the traversal kernels (no reference counterpart: the reference launches
  * one thread per ray in blocks of 256, kernel.mojo:649-662). Results do not depend on it.
  *   persistent  : 0 = one lane per ray; 1 = persistent lanes refilled from an atomic ray
@@ -272,9 +276,7 @@ int gz_gpu_expand_hits_device(void *handle, const struct GzHit *d_hits, const fl
  *   ldsStack    : stack entries kept in LDS per lane (0, 8 or 16; the rest in private memory);
  *   refillLanes : idle lanes (1..64) that trigger a refill of a wave's lanes (modes 1, 3);
  *   gridScale   : persistent grid = gridScale x the blocks resident per CU x CUs (0 = 1);
- *   chunk       : rays a wave takes from a counter per atomic (modes 1, 3; 1..4096); also the
- *                 queue entries a wave of the MIS full wavefront's path-ray kernel takes per
- *                 atomic (default 128);
+ *   chunk       : rays a wave takes from a counter per atomic (modes 1, 3; 1..4096);
  *   binMinRays  : batches of at least this many rays (and at least 1) are traced in the order of
  *                 their origin's cell in a 16^3 grid over the scene box (a counting sort on the
  *                 device, into storage the handle keeps per stream: 34 bytes per ray plus 16 KiB
@@ -284,7 +286,10 @@ int gz_gpu_expand_hits_device(void *handle, const struct GzHit *d_hits, const fl
  *   recordTimes : 1 = record HIP events around the binning and the traversal kernel of each
  *                 launch, for gz_gpu_trace_times (0 = none).
  * Until a configuration is set, batches below 2^22 rays run in mode 0, in the given order but for scenes of
- * more than 2^18 primitives from 3 x 2^20 rays on (more than 2^21 primitives: from 2^21 rays on). */
+ * more than 2^18 primitives from 3 x 2^20 rays on (more than 2^21 primitives: from 2^21 rays on), and larger
+ * ones as {3, 16, 32, 1, 128, 2^18}; gz_gpu_get_trace_config then returns these values with reserved =
+ * GZ_LAUNCH_BY_SIZE. Setting them so (recordTimes either way) goes back to that rule; with any other values
+ * GZ_LAUNCH_BY_SIZE is not read and the configuration holds for every batch. */
 struct GzTraceConfig {
         int32_t persistent;
         int32_t ldsStack;
@@ -436,11 +441,13 @@ int gz_gpu_mis_trace_device(void *handle, struct GzPath *d_paths, int64_t count,
  *               remaining bounces in one launch (a lane per path), in place of one launch
  *               sequence per level for the few paths that Russian roulette leaves (the
  *               adjoint's replay drains from the same level);
- *   reserved  : zero.
- * Until gz_gpu_set_mis_launch sets one, a handle uses {1, 256, 1, 256, 3} if every material is
- * diffuse and it has at most 65536 primitives, else {3, 256, 1, 64, 3} (gz_gpu_get_mis_launch
- * returns the one in use); up to 2^19 paths (2^20 for the latter) a forward trace then runs each path
- * whole, in one launch, and keeps no queues. */
+ *   reserved  : zero, but for reserved[0] as below.
+ * Until gz_gpu_set_mis_launch sets one, a handle's launch is {1, 256, 1, 256, 3} if every material is
+ * diffuse and it has at most 65536 primitives, else {3, 256, 1, 64, 3}, and it goes by size: up to 2^19
+ * paths (2^20 for the latter) a forward trace runs each path whole, in one launch, and keeps no queues, and
+ * above that the former takes 128 queue entries a wave. gz_gpu_get_mis_launch then returns that launch with
+ * reserved[0] = GZ_LAUNCH_BY_SIZE. Setting either of the two so goes back to the default; with any other
+ * values GZ_LAUNCH_BY_SIZE is not read and the launch holds for every count. */
 struct GzMisLaunch {
         int32_t queued;
         int32_t block;
@@ -619,7 +626,8 @@ int gz_batch_info(void *batch, struct GzBatchInfo *info);
  * the others with the bounce kernel, level by level. The default is {3, 256, 1, 64, 3} when some
  * scene's default is the wavefront, else {1, 256, 1, 256, 3}; until one is set, batches
  * whose rounds hold at most 2^20 paths of wavefront scenes and 3 x 2^20 in all (2^19 without a wavefront
- * scene) run each path whole, in one launch. */
+ * scene) run each path whole, in one launch. Either of the two with reserved[0] = GZ_LAUNCH_BY_SIZE goes back
+ * to the default, as for gz_gpu_set_mis_launch. */
 int gz_batch_set_launch(void *batch, const struct GzMisLaunch *launch);
 /* Renders every path of every scene once and adds it to the scenes' films, asynchronously on
  * `stream`. Each round is the same launch sequence (camera rays, device path queues per bounce
