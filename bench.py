@@ -321,7 +321,7 @@ def path_leg(args, dev, stream, host: dict, run_cpu: bool) -> dict:
                           "unit": "GB/s", "frac": round(algo / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)},
              "image_mean_rgb": [round(float(x), 5) for x in img.reshape(-1, 3).mean(0)],
              "film_zero_weight_pixels": int(film.bad.item()), "lanes": rnd.lanes,
-             "launch": describe(timings)[0], "launch_ms": describe(timings)}
+             "launch": describe({best: timings[best]})[0], "launch_ms": describe(timings)}
     log(f"path leg: {res_d['path_samples_per_s'] / 1e6:.2f} M path samples/s, {ms:.2f} ms/frame, "
         f"{res_d['bounces_per_path']} bounces/path, {res_d['bytes_per_path']} B/path")
     if run_cpu:
@@ -407,7 +407,7 @@ def full_path_leg(args, dev, stream, host: dict, run_cpu: bool) -> dict:
            "image_mean_rgb": [round(float(x), 5) for x in img.reshape(-1, 3).mean(0)],
            "film_zero_weight_pixels": int(film.bad.item()),
            "lanes": rnd.lanes, "lane_bounds": rnd.bounds,
-           "launch": describe(timings)[0], "launch_ms": describe(timings)}
+           "launch": describe({best: timings[best]})[0], "launch_ms": describe(timings)}
     log(f"full path leg: {res['path_samples_per_s'] / 1e6:.2f} M path samples/s, {ms:.1f} ms/frame, "
         f"{res['bounces_per_path']} bounces/path")
     if run_cpu:
@@ -522,7 +522,7 @@ def batch_leg(args, dev, stream, host: dict, run_cpu: bool) -> dict:
     from gonzales_amd import abi
     solo = abi.GZ_BATCH_SOLO_PATHS if args.batch_solo_paths is None else args.batch_solo_paths
     batch = SceneBatch(entries, round_paths=args.batch_round_paths, solo_paths=solo)
-    batch.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued)
+    batch.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued, best.by_size)
     info = batch.info()
     n = info.totalPaths
     batch.render(True)  # capture + warm-up
@@ -582,7 +582,7 @@ def batch_leg(args, dev, stream, host: dict, run_cpu: bool) -> dict:
         if len(idx) == 0:
             continue
         sub = SceneBatch([entries[k] for k in idx], round_paths=args.batch_round_paths, solo_paths=solo)
-        sub.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued)
+        sub.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued, best.by_size)
         sub.render(True)
         torch.cuda.synchronize()
         a.record(stream)
@@ -611,7 +611,7 @@ def batch_leg(args, dev, stream, host: dict, run_cpu: bool) -> dict:
            "tris_per_path": round(st[1] / n, 2), "bytes_per_path": round(algo / n, 1),
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4)},
-           "host_scene_build_s": round(t_build, 2), "launch": describe(timings)[0], "launch_ms": describe(timings)}
+           "host_scene_build_s": round(t_build, 2), "launch": describe({best: timings[best]})[0], "launch_ms": describe(timings)}
     log(f"batch leg: {n / (ms * 1e-3) / 1e6:.1f} M path samples/s over {n} samples, {ms:.0f} ms "
         f"(one scene at a time {seq_ms:.0f} ms), {info.rounds} rounds, {algo / n:.0f} B/path")
     batch.close()
@@ -935,7 +935,7 @@ def main() -> int:
         log(f"autotuned launch config: {best}")
     binned = best.bin_min_rays > 0 and n >= best.bin_min_rays
     bh.set_trace_config(best.persistent, best.lds_stack, best.refill_lanes, best.grid_scale, best.chunk,
-                        best.bin_min_rays, record_times=1)
+                        best.bin_min_rays, record_times=1, by_size=best.by_size)
 
     # Work counts for the algorithmic bytes (untimed counting pass).
     bh.closest_device(d_rays, d_tmax, d_hits, d_stats)
@@ -1021,7 +1021,7 @@ def main() -> int:
         extra["coherent_anyhit_mrays_per_s"] = round(nc / (ms_ca * 1e-3) / 1e6, 2)
         extra["coherent_launch_config"] = describe({cbest: 0.0})[0]
         bh.set_trace_config(best.persistent, best.lds_stack, best.refill_lanes, best.grid_scale, best.chunk,
-                            best.bin_min_rays, record_times=1)
+                            best.bin_min_rays, record_times=1, by_size=best.by_size)
         extra["device_build"] = device_build_leg(args, bh, d_rays, d_tmax, n, stream, mrays)
         # End to end through host buffers (H2D + trace + Intersection_C expansion + D2H), 1M rays.
         # (steady state: the first call grows the staging buffers and is not timed)

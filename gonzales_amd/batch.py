@@ -13,6 +13,7 @@ import ctypes
 from dataclasses import dataclass
 
 from . import abi
+from .autotune import fastest, first_again
 from .camera import DeviceFilm, PerspectiveCamera
 from .integrator import VolumePathIntegrator
 
@@ -102,17 +103,17 @@ class BatchLaunch:
     chunk: int = 256
     drain_level: int = 3
     queued: int = 1
+    by_size: int = 0  # 1 with a default launch's values: the choice by scenes and round size
 
 
 BATCH_CANDIDATES = (
+    BatchLaunch(by_size=1),
     BatchLaunch(256, 1, 64, 3, 3),
     BatchLaunch(256, 1, 256, 3, 3),
     BatchLaunch(256, 1, 64, 2, 3),
     BatchLaunch(256, 1, 64),
     BatchLaunch(256, 1, 256),
     BatchLaunch(256, 1, 1024),
-    BatchLaunch(256, 2, 256),
-    BatchLaunch(128, 1, 256),
     BatchLaunch(256, 1, 256, 0),
 )
 
@@ -124,8 +125,8 @@ def autotune_batch(batch: SceneBatch, candidates=BATCH_CANDIDATES, reps: int = 1
 
     s = torch.cuda.current_stream()
     timings = {}
-    for cfg in candidates:
-        batch.set_launch(cfg.block, cfg.grid_scale, cfg.chunk, cfg.drain_level, cfg.queued)
+    for cfg in first_again(candidates):
+        batch.set_launch(cfg.block, cfg.grid_scale, cfg.chunk, cfg.drain_level, cfg.queued, cfg.by_size)
         batch.render(True)  # captures the graph for this shape
         torch.cuda.synchronize()
         a = torch.cuda.Event(enable_timing=True)
@@ -135,9 +136,10 @@ def autotune_batch(batch: SceneBatch, candidates=BATCH_CANDIDATES, reps: int = 1
             batch.render(True)
         b.record(s)
         torch.cuda.synchronize()
-        timings[cfg] = a.elapsed_time(b) / reps
-    best = min(timings, key=timings.get)
-    batch.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued)
+        ms = a.elapsed_time(b) / reps
+        timings[cfg] = min(ms, timings.get(cfg, ms))
+    best = fastest(timings)
+    batch.set_launch(best.block, best.grid_scale, best.chunk, best.drain_level, best.queued, best.by_size)
     batch.clear_films()
     return best, timings
 
