@@ -572,10 +572,11 @@ static MisQueue *full_queue(MisQueues *&owner, hipStream_t stream, size_t count,
 // Grid of a persistent queue kernel: gridScale x the blocks resident per CU x CUs, and no more
 // blocks than the first level has chunks of work for.
 template <typename K>
-static unsigned queue_grid(Scene *s, K kern, int block, int64_t count, unsigned chunk) {
+static unsigned queue_grid(const Scene *s, const GzMisLaunch &c, K kern, int64_t count) {
+        const int block = c.block;
+        const unsigned chunk = (unsigned)c.chunk;
         int perCU = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kern, block, 0) != hipSuccess || perCU < 1) perCU = 1;
-        const GzMisLaunch &c = s->misLaunch;
         const int64_t want = (int64_t)s->cuCount * perCU * (c.gridScale > 0 ? c.gridScale : 1);
         const int64_t wavesPerBlock = block / 64;
         const int64_t need = ((count + chunk - 1) / chunk + wavesPerBlock - 1) / wavesPerBlock;
@@ -962,15 +963,14 @@ bool gz::mis_args(Scene *s, const GzMisParams *params, int *err, MisArgs &a) {
 // the counters, then one persistent launch per level. `launch(level, grid, qin, qout, ctl)`
 // enqueues one level's kernel.
 template <typename K, typename Launch>
-static int queued_levels(Scene *s, MisQueues *&owner, K kern, int64_t count, int maxDepth, hipStream_t st,
-                         const char *who, Launch &&launch,
+static int queued_levels(Scene *s, const GzMisLaunch &c, MisQueues *&owner, K kern, int64_t count, int maxDepth,
+                         hipStream_t st, const char *who, Launch &&launch,
                          const std::function<void(unsigned, const int *, unsigned *)> &drain = {}) {
         const int levels = maxDepth + 2;
         MisQueue *q = mis_queue(owner, st, (size_t)count, levels);
         if (!q) return GZ_E_ALLOC;
-        const GzMisLaunch &c = s->misLaunch;
         const unsigned chunk = (unsigned)c.chunk;
-        const unsigned grid = queue_grid(s, kern, c.block, count, chunk);
+        const unsigned grid = queue_grid(s, c, kern, count);
         hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(256), 0, st, q->ctl, levels);
         if (!hip_ok(hipGetLastError(), who)) return GZ_E_HIP;
         for (int level = 0; level <= maxDepth; ++level) {
@@ -1047,10 +1047,11 @@ static MisRecord record_at(void *base, int64_t count, int levels) {
 
 // queues: the queue storage to use (null: the handle's own); err: the flag traversal overflows
 // raise (null: the handle's, per stream); rec: a replay record to fill (full wavefront levels
-// below the drain level; every other entry stays marked as not traced).
+// below the drain level; every other entry stays marked as not traced); own: the launch of this call
+// (null: the handle's).
 static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisParams *params,
                       GzPathStats *d_stats, void *stream, bool toEnd, const char *who, MisQueues **queues = nullptr,
-                      int *err = nullptr, const MisRecord *rec = nullptr) {
+                      int *err = nullptr, const MisRecord *rec = nullptr, const GzMisLaunch *own = nullptr) {
         clear_error();
         if (!handle || count < 0 || (count > 0 && !d_paths)) {
                 set_error("%s: bad arguments", who);
@@ -1082,7 +1083,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
         uint32_t *stats = reinterpret_cast<uint32_t *>(d_stats);
         const bool all = !s->mis->allDiffuse;
         const int bset = mis_bsdf_set(s);
-        const LaunchChoice lc = launch_for(s, count, rec != nullptr);
+        const LaunchChoice lc = own ? LaunchChoice{*own, false} : launch_for(s, count, rec != nullptr);
         if (toEnd && lc.launch.queued == 3) {
                 if (count > 0x7fffffffLL) {
                         set_error("%s: %lld paths exceed one queue (2^31 - 1)", who, (long long)count);
@@ -1091,7 +1092,7 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 const int levels = params->maxDepth + 2;
                 MisQueue *q = full_queue(owner, st, (size_t)count, levels);
                 if (!q) return GZ_E_ALLOC;
-                const GzMisLaunch &c = s->misLaunch;
+                const GzMisLaunch &c = lc.launch;
                 auto ktrace = d_stats ? k_wf_rays<0, true> : k_wf_rays<0, false>;
                 auto kany = d_stats ? k_wf_rays<1, true> : k_wf_rays<1, false>;
                 auto kclose = d_stats ? k_wf_rays<2, true> : k_wf_rays<2, false>;
@@ -1104,9 +1105,9 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 const int classes = !all ? 1 : 3;
                 const unsigned tgrid = rays_grid(s, count);
                 const unsigned chunk = (unsigned)c.chunk;
-                const unsigned gd = queue_grid(s, kd, c.block, count, chunk);
-                const unsigned ga = queue_grid(s, ka, c.block, count, chunk);
-                const unsigned gn = queue_grid(s, kn, c.block, count, chunk);
+                const unsigned gd = queue_grid(s, c, kd, count);
+                const unsigned ga = queue_grid(s, c, ka, count);
+                const unsigned gn = queue_grid(s, c, kn, count);
                 const unsigned sgrid = (unsigned)std::max<int64_t>(
                         1, std::min<int64_t>((int64_t)s->cuCount * 8, (count + kMisBlock - 1) / kMisBlock));
                 const unsigned spgrid = split_grid(s, count);
@@ -1164,15 +1165,15 @@ static int mis_launch(void *handle, GzPath *d_paths, int64_t count, const GzMisP
                 const int levels = params->maxDepth + 2;
                 MisQueue *q = wf_queue(owner, st, (size_t)count, levels);
                 if (!q) return GZ_E_ALLOC;
-                const GzMisLaunch &c = s->misLaunch;
+                const GzMisLaunch &c = lc.launch;
                 auto ktrace = d_stats ? k_wf_rays<0, true> : k_wf_rays<0, false>;
                 auto kd = d_stats ? k_wf_shade<true, 0> : k_wf_shade<false, 0>;
                 auto ka = d_stats ? (bset == kBsdfNoLayer ? k_wf_shade<true, 2> : k_wf_shade<true, 1>)
                                   : (bset == kBsdfNoLayer ? k_wf_shade<false, 2> : k_wf_shade<false, 1>);
                 const unsigned tgrid = rays_grid(s, count);
                 const unsigned chunk = (unsigned)c.chunk;
-                const unsigned gd = queue_grid(s, kd, c.block, count, chunk);
-                const unsigned ga = queue_grid(s, ka, c.block, count, chunk);
+                const unsigned gd = queue_grid(s, c, kd, count);
+                const unsigned ga = queue_grid(s, c, ka, count);
                 auto kdrain = d_stats ? pick_set(bset, k_mis_drain<true, 0>, k_mis_drain<true, 1>, k_mis_drain<true, 2>)
                                       : pick_set(bset, k_mis_drain<false, 0>, k_mis_drain<false, 1>, k_mis_drain<false, 2>);
                 hipLaunchKernelGGL(k_wf_clear, dim3(1), dim3(256), 0, st, q->wctl, levels);
@@ -1335,9 +1336,11 @@ extern "C" int gz_gpu_mis_trace_stats_device(void *handle, GzPath *d_paths, int6
 // 2.12 / 2.09, 4.2M 5.6 / 5.1, 8.4M 10.7 / 9.5; tracing its rays again: 2.1M 3.6 / 3.2, 8.4M 17.9 / 15.5.
 static bool replay_shares_head(int64_t count) { return count > (int64_t)3 << 19; }
 
-// The adjoint replay; rec: the forward pass's replay record (null: every ray is traced again).
+// The adjoint replay; rec: the forward pass's replay record (null: every ray is traced again); own: the launch
+// of this call (null: the handle's).
 static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adjoint, int64_t count,
-                       const GzMisParams *params, double *d_grad, void *stream, const MisRecord *rec) {
+                       const GzMisParams *params, double *d_grad, void *stream, const MisRecord *rec,
+                       const GzMisLaunch *own = nullptr) {
         clear_error();
         if (!handle || count < 0 || (count > 0 && (!d_paths || !d_adjoint || !d_grad))) {
                 set_error("gz_gpu_mis_adjoint_device: bad arguments");
@@ -1366,7 +1369,8 @@ static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adj
                 adj.recCount = count;
         }
         refresh_default_launch(s);
-        if (s->misLaunch.queued) {
+        const GzMisLaunch c = own ? *own : s->misLaunch;
+        if (c.queued) {
                 if (count > 0x7fffffffLL) {
                         set_error("gz_gpu_mis_adjoint_device: %lld paths exceed one queue (2^31 - 1)", (long long)count);
                         return GZ_E_INVALID;
@@ -1374,15 +1378,15 @@ static int mis_adjoint(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adj
                 const int bset = mis_bsdf_set(s);
                 auto kern = pick_set(bset, k_mis_adjoint_queue<0>, k_mis_adjoint_queue<1>, k_mis_adjoint_queue<2>);
                 auto kdrain = pick_set(bset, k_mis_adjoint_drain<0>, k_mis_adjoint_drain<1>, k_mis_adjoint_drain<2>);
-                const int block = s->misLaunch.block;
+                const int block = c.block;
                 const bool shared = replay_shares_head(count);
                 std::function<void(unsigned, const int *, unsigned *)> drain;
-                if (s->misLaunch.drainLevel > 0)
+                if (c.drainLevel > 0)
                         drain = [&](unsigned grid, const int *qin, unsigned *n) {
                                 hipLaunchKernelGGL(kdrain, dim3(grid), dim3(block), 0, st, a, d_paths, qin, n, adj);
                         };
                 return queued_levels(
-                        s, s->misQueues, kern, count, params->maxDepth, st, "MIS adjoint launch",
+                        s, c, s->misQueues, kern, count, params->maxDepth, st, "MIS adjoint launch",
                         [&](int level, unsigned grid, const int *qin, int *qout, QueueLevel *ctl, unsigned chunk) {
                                 hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, a, d_paths, (unsigned)count, qin,
                                                    qout, ctl, level, chunk, adj, shared);
@@ -1407,13 +1411,37 @@ extern "C" int64_t gz_mis_record_bytes(int64_t count, int32_t levels) {
         return count * (int64_t)levels * (int64_t)(2 * sizeof(GzHit) + 1);
 }
 
+// Whether (record, levels, launch) are what a recorded trace or replay takes.
+static bool record_ok(const void *d_record, int32_t levels, int64_t count, const GzMisLaunch *launch, const char *who) {
+        clear_error();
+        if (levels < 0 || levels > kMaxRecordLevels || (levels > 0 && count > 0 && !d_record)) {
+                set_error("%s: need 0 <= levels <= %d and a record", who, kMaxRecordLevels);
+                return false;
+        }
+        return !launch || launch_ok(*launch, who);
+}
+
+extern "C" int gz_gpu_mis_trace_record_launch_device(void *handle, GzPath *d_paths, int64_t count,
+                                                     const GzMisParams *params, const GzMisLaunch *launch,
+                                                     void *d_record, int32_t levels, void *stream) {
+        const char *who = "gz_gpu_mis_trace_record_launch_device";
+        if (!record_ok(d_record, levels, count, launch, who)) return GZ_E_INVALID;
+        const MisRecord rec = record_at(d_record, count, levels);
+        return mis_launch(handle, d_paths, count, params, nullptr, stream, true, who, nullptr, nullptr, &rec, launch);
+}
+
+extern "C" int gz_gpu_mis_adjoint_record_launch_device(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adjoint,
+                                                       int64_t count, const GzMisParams *params,
+                                                       const GzMisLaunch *launch, double *d_grad, const void *d_record,
+                                                       int32_t levels, void *stream) {
+        if (!record_ok(d_record, levels, count, launch, "gz_gpu_mis_adjoint_record_launch_device")) return GZ_E_INVALID;
+        const MisRecord rec = record_at(const_cast<void *>(d_record), count, levels);
+        return mis_adjoint(handle, d_paths, d_adjoint, count, params, d_grad, stream, &rec, launch);
+}
+
 extern "C" int gz_gpu_mis_trace_record_device(void *handle, GzPath *d_paths, int64_t count, const GzMisParams *params,
                                               void *d_record, int32_t levels, void *stream) {
-        if (levels < 0 || levels > kMaxRecordLevels || (levels > 0 && count > 0 && !d_record)) {
-                clear_error();
-                set_error("gz_gpu_mis_trace_record_device: need 0 <= levels <= %d and a record", kMaxRecordLevels);
-                return GZ_E_INVALID;
-        }
+        if (!record_ok(d_record, levels, count, nullptr, "gz_gpu_mis_trace_record_device")) return GZ_E_INVALID;
         const MisRecord rec = record_at(d_record, count, levels);
         return mis_launch(handle, d_paths, count, params, nullptr, stream, true, "gz_gpu_mis_trace_record_device",
                           nullptr, nullptr, &rec);
@@ -1422,11 +1450,7 @@ extern "C" int gz_gpu_mis_trace_record_device(void *handle, GzPath *d_paths, int
 extern "C" int gz_gpu_mis_adjoint_record_device(void *handle, GzPath *d_paths, const GzPathAdjoint *d_adjoint,
                                                 int64_t count, const GzMisParams *params, double *d_grad,
                                                 const void *d_record, int32_t levels, void *stream) {
-        if (levels < 0 || levels > kMaxRecordLevels || (levels > 0 && count > 0 && !d_record)) {
-                clear_error();
-                set_error("gz_gpu_mis_adjoint_record_device: need 0 <= levels <= %d and a record", kMaxRecordLevels);
-                return GZ_E_INVALID;
-        }
+        if (!record_ok(d_record, levels, count, nullptr, "gz_gpu_mis_adjoint_record_device")) return GZ_E_INVALID;
         const MisRecord rec = record_at(const_cast<void *>(d_record), count, levels);
         return mis_adjoint(handle, d_paths, d_adjoint, count, params, d_grad, stream, &rec);
 }

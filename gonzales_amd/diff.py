@@ -1,10 +1,10 @@
 """Differentiable rendering: a torch.autograd.Function over the GPU MIS integrator whose backward
 pass is the path-replay adjoint kernel (gz_gpu_mis_adjoint_device).
 
-By default the forward pass also keeps a replay record in HBM (gz_gpu_mis_trace_record_device: each
+By default the forward pass also keeps a replay record in HBM (gz_gpu_mis_trace_record_launch_device: each
 path's closest hit, BSDF-ray hit and shadow visibility for the wavefront levels, 33 B per path and
 level), and the backward pass replays the paths from it instead of tracing their rays again
-(gz_gpu_mis_adjoint_record_device); the gradients are the same.
+(gz_gpu_mis_adjoint_record_launch_device); the gradients are the same.
 
 Parameters are the reflectance of diffuse materials and the (isotropic) roughness of conductor
 materials of the scene's GzMaterial table. forward renders the image (camera -> bounces -> film)
@@ -25,8 +25,9 @@ from .integrator import MisOptions, VolumePathIntegrator
 
 class DiffRenderer:
     """Renders a full-frame camera (no crop) with the parameters written into the material table.
-    record (default): keep the forward pass's replay record and replay from it; this sets the scene
-    handle's launch to the full wavefront without a drain level (every level recorded)."""
+    record (default): keep the forward pass's replay record and replay from it. Both passes then run under
+    the full wavefront, with a drain level by the frame's path count (the levels before it are recorded), as
+    long as no launch is set on the scene handle after construction; the handle's own launch is left alone."""
 
     def __init__(self, bh, camera: PerspectiveCamera, materials: np.ndarray, options: MisOptions, sky=None,
                  device="cuda", record: bool = True):
@@ -46,14 +47,16 @@ class DiffRenderer:
         self.record = record
         self.d_record = None
         self.recorded_levels = 0  # levels the last render recorded (0: none; backward traces every ray)
-        if record:
-            # The full wavefront, recording every level it runs (the backward then traces nothing there).
-            # From 2^20 paths on every level; below, the last levels hold too few paths to fill the chip
-            # twice each, and a drain from level 2 (up to 2^18 paths) or 3 is faster for both passes although
-            # it records nothing. Step of a room with 50K triangles, depth 5, drain 0 / 2 / 3 in ms: 16K paths
-            # 1.51 / 1.34 / 1.46, 65K 2.21 / 1.88 / 2.09, 262K 2.72 / 2.27 / 2.52, 1M 4.59 / 5.46 / 4.29, 4.2M
-            # 12.9 / 17.7 / 13.3.
-            self.integrator.set_launch(3, 256, 1, 64, 2 if n <= 1 << 18 else 3 if n <= 1 << 20 else 0)
+        # The full wavefront, recording every level it runs (the backward then traces nothing there). Above
+        # 2^20 paths every level; up to that the last levels hold too few paths to fill the chip
+        # twice each, and a drain from level 2 (up to 2^18 paths) or 3 is faster for both passes although
+        # it records nothing. Step of a room with 50K triangles, depth 5, drain 0 / 2 / 3 in ms: 16K paths
+        # 1.51 / 1.34 / 1.46, 65K 2.21 / 1.88 / 2.09, 262K 2.72 / 2.27 / 2.52, 1M 4.59 / 5.46 / 4.29, 4.2M
+        # 12.9 / 17.7 / 13.3.
+        drain = 2 if n <= 1 << 18 else 3 if n <= 1 << 20 else 0
+        self.launch = abi.GzMisLaunch(3, 256, 1, 64, drain) if record else None
+        self._handle_launch = bytes(self.integrator._launch())
+        self._rendered_launch = None  # the launch of the last render (None: the handle's)
 
     def set_parameters(self, albedo=None, roughness=None) -> None:
         """albedo: (M, 3) reflectances (used where the material is diffuse); roughness: (M,)
@@ -75,34 +78,42 @@ class DiffRenderer:
         import torch
         self.camera.paths_device(self.d_start)
         self.d_paths.copy_(self.d_start)
-        levels = self._record_levels() if self.record else 0
-        if levels > 0:
+        launch = self._own_launch()
+        levels = self._record_levels(launch) if self.record else 0
+        if launch or levels > 0:
             lib = abi.load()
             need = int(lib.gz_mis_record_bytes(self.n, levels))
-            if self.d_record is None or self.d_record.numel() < need:
+            if levels > 0 and (self.d_record is None or self.d_record.numel() < need):
                 self.d_record = None
                 self.d_record = torch.empty(need, dtype=torch.uint8, device=self.device)
-            abi.check(lib.gz_gpu_mis_trace_record_device(self.bh.handle, abi.ptr(self.d_paths), self.n,
-                                                         ctypes.byref(self.options.params()), abi.ptr(self.d_record),
-                                                         levels, abi.stream_ptr(None)),
-                      "gz_gpu_mis_trace_record_device")
+            abi.check(lib.gz_gpu_mis_trace_record_launch_device(
+                self.bh.handle, abi.ptr(self.d_paths), self.n, ctypes.byref(self.options.params()),
+                ctypes.byref(launch) if launch else None, abi.ptr(self.d_record) if levels > 0 else None, levels,
+                abi.stream_ptr(None)), "gz_gpu_mis_trace_record_launch_device")
         else:
             self.integrator.trace(self.d_paths)
         self.recorded_levels = levels
+        self._rendered_launch = launch
         self.film.clear()
         self.film.add(self.d_paths, self.n)
         img = self.film.resolve()
         c = self.camera.c
         return img.view(c.resY, c.resX, 3).clone()
 
-    def _record_levels(self) -> int:
+    def _own_launch(self):
+        """The launch of this renderer's calls: its own, if it was made to record, while the handle has none set
+        (or the one it had at construction), else None, the handle's."""
+        c = self.integrator._launch()
+        return self.launch if c.reserved[0] == abi.GZ_LAUNCH_BY_SIZE or bytes(c) == self._handle_launch else None
+
+    def _record_levels(self, launch) -> int:
         """Bounce levels the forward pass can record: those the full wavefront launch runs level by
         level (below its drain level); none for the other launch shapes."""
-        queued, _, _, _, drain = self.integrator.launch()
-        if queued != 3:
+        c = launch or self.integrator._launch()
+        if c.queued != 3:
             return 0
         levels = self.options.max_depth + 1
-        return min(levels, drain) if drain > 0 else levels
+        return min(levels, c.drainLevel) if c.drainLevel > 0 else levels
 
     def path_radiance(self):
         """(n, 3) radiance of each path sample of the last render (a strided view of the records)."""
@@ -126,14 +137,12 @@ class DiffRenderer:
         grad = torch.zeros(len(self.materials) * 4, dtype=torch.float64, device=self.device)
         self.d_paths.copy_(self.d_start)
         prm = self.options.params()
-        if self.recorded_levels > 0:
-            abi.check(abi.load().gz_gpu_mis_adjoint_record_device(
-                self.bh.handle, abi.ptr(self.d_paths), abi.ptr(adj), self.n, ctypes.byref(prm), abi.ptr(grad),
-                abi.ptr(self.d_record), self.recorded_levels, None), "gz_gpu_mis_adjoint_record_device")
-        else:
-            abi.check(abi.load().gz_gpu_mis_adjoint_device(self.bh.handle, abi.ptr(self.d_paths), abi.ptr(adj),
-                                                            self.n, ctypes.byref(prm), abi.ptr(grad), None),
-                      "gz_gpu_mis_adjoint_device")
+        launch = self._rendered_launch if self.recorded_levels > 0 else self._own_launch()
+        abi.check(abi.load().gz_gpu_mis_adjoint_record_launch_device(
+            self.bh.handle, abi.ptr(self.d_paths), abi.ptr(adj), self.n, ctypes.byref(prm),
+            ctypes.byref(launch) if launch else None, abi.ptr(grad),
+            abi.ptr(self.d_record) if self.recorded_levels > 0 else None, self.recorded_levels, None),
+            "gz_gpu_mis_adjoint_record_launch_device")
         grad = grad.view(-1, 4)
         return grad[:, :3].clone(), grad[:, 3].clone()
 

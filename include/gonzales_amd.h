@@ -517,6 +517,16 @@ int gz_gpu_mis_trace_record_device(void *handle, struct GzPath *d_paths, int64_t
 int gz_gpu_mis_adjoint_record_device(void *handle, struct GzPath *d_paths, const struct GzPathAdjoint *d_adjoint,
                                      int64_t count, const struct GzMisParams *params, double *d_grad,
                                      const void *d_record, int32_t levels, void *stream);
+/* The same two calls under a launch of their own (NULL: the handle's): the handle's launch, which other
+ * renderers of the scene use, is neither read nor changed. Pass both calls the same launch; levels may be 0 (no
+ * record). */
+int gz_gpu_mis_trace_record_launch_device(void *handle, struct GzPath *d_paths, int64_t count,
+                                          const struct GzMisParams *params, const struct GzMisLaunch *launch,
+                                          void *d_record, int32_t levels, void *stream);
+int gz_gpu_mis_adjoint_record_launch_device(void *handle, struct GzPath *d_paths,
+                                            const struct GzPathAdjoint *d_adjoint, int64_t count,
+                                            const struct GzMisParams *params, const struct GzMisLaunch *launch,
+                                            double *d_grad, const void *d_record, int32_t levels, void *stream);
 
 /* ---------------------------------------------------------------------------------------- */
 /* Camera samples, primary rays and film (Core/Tile.swift:27-59, :170-219; Core/Film.swift).  */

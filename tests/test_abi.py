@@ -87,3 +87,16 @@ def test_zsobol_rejects_bad_patterns():
     assert rc == abi.GZ_E_INVALID and "pattern" in abi.last_error()
     rc = lib.gz_zsobol_tile_device(ctypes.byref(p), 0, 0, 4, 4, 4, 1024, bad.ctypes.data, 1, None, 0, None)
     assert rc == abi.GZ_E_INVALID
+
+
+def test_recorded_trace_and_replay_check_their_launch():
+    lib = abi.load()
+    ok, bad = abi.GzMisLaunch(3, 256, 1, 64, 0), abi.GzMisLaunch(3, 100, 1, 64, 0)
+    trace, adjoint = lib.gz_gpu_mis_trace_record_launch_device, lib.gz_gpu_mis_adjoint_record_launch_device
+    for launch, levels, said in ((bad, 0, "block 100"), (ok, -1, "levels"), (ok, 1 << 20, "levels"), (ok, 0, "bad arguments"),
+                                 (None, 0, "bad arguments")):
+        p = ctypes.byref(launch) if launch else None
+        assert trace(None, None, 0, None, p, None, levels, None) == abi.GZ_E_INVALID
+        assert said in abi.last_error()
+        assert adjoint(None, None, None, 0, None, p, None, None, levels, None) == abi.GZ_E_INVALID
+        assert said in abi.last_error()

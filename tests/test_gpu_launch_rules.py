@@ -128,3 +128,45 @@ def test_replay_of_large_frames_equals_the_full_relaunch(gpu, res, spp):
             assert float(y.abs().max()) > 0
             assert float((x - y).abs().max()) <= 5e-9 * float(y.abs().max())
     bh.free()
+
+
+def test_diff_renderers_of_two_sizes_on_one_handle(gpu):
+    """Each renderer runs under its own launch whatever others of the same hierarchy are made between, and the
+    handle's launch stays the default: a large frame records every level, a small one up to its drain level,
+    with the images and gradients of renderers of their own hierarchies. A launch set on the handle holds for both."""
+    import torch
+    from gonzales_amd.camera import Film, PerspectiveCamera, pbrt_transform
+    from gonzales_amd.diff import DiffRenderer
+
+    def make(bh, gz, res, spp):
+        cam = PerspectiveCamera(pbrt_transform([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, -1, 0, 0, -1, 6.8, 1]), 19.5, Film(*res), spp, 0)
+        opt = MisOptions(max_depth=3, zsobol_seed=cam.c.zsSeed, log2_spp=cam.c.zsLog2Spp, base4_digits=cam.c.zsBase4Digits)
+        return DiffRenderer(bh, cam, gz, opt)
+
+    def step(r):
+        img = r.render()
+        return (img, *r.backward(2 * img), r.recorded_levels)
+
+    def scene():
+        bh, gz, _, _ = scenes.inverse_rendering_scene(subdivisions=3, n_params=8)
+        bh.upload_to_gpu()
+        return bh, gz
+
+    sizes = (((512, 257), 8), ((64, 48), 4), ((512, 200), 8))
+    bh, gz = scene()
+    shared = [make(bh, gz, *size) for size in sizes]
+    got = [step(r) for r in shared]
+    assert [g[3] for g in got] == [4, 2, 3]
+    assert shared[0].integrator.launch_by_size()
+    for size, g in zip(sizes, got):
+        bh2, gz2 = scene()
+        img, ga, gr, levels = step(make(bh2, gz2, *size))
+        assert torch.equal(img, g[0]) and levels == g[3]
+        for x, y in ((ga, g[1]), (gr, g[2])):
+            assert float((x - y).abs().max()) <= 5e-9 * float(y.abs().max())
+        bh2.free()
+    shared[0].integrator.set_launch(3, 256, 1, 64, 1)
+    assert [step(r)[3] for r in shared] == [1, 1, 1]
+    shared[0].integrator.reset_launch()
+    assert [step(r)[3] for r in shared] == [4, 2, 3]
+    bh.free()
