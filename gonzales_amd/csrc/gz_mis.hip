@@ -133,12 +133,12 @@ __device__ __forceinline__ void queue_run(unsigned nin, const int *__restrict__ 
 // bounce (bounce_rest) over one class queue: the diffuse kernel is the small one (4 waves/SIMD),
 // only the other class pays for the 256-register kernel. Survivors go to the next level's queue.
 struct WfLevel {
-        unsigned qn, qhead;    // the level's queue (appended by the previous level's shade kernels)
+        unsigned qn;           // the level's queue (appended by the previous level's shade kernels)
         unsigned dn, dhead;    // diffuse class
         unsigned an, ahead;    // other BSDFs
         unsigned sn, mn;       // shadow rays and BSDF rays (full wavefront; taken by static striding)
         unsigned nn;           // BSDFs but the layered one (full wavefront)
-        unsigned pad[7];
+        unsigned pad[8];
 };
 static_assert(sizeof(WfLevel) == 64, "WfLevel");
 
