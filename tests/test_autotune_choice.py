@@ -16,4 +16,5 @@ def test_the_default_stays_unless_another_is_faster_than_the_noise():
     default, other = MisLaunch(1, 256, 1, 256, 3, by_size=1), MisLaunch(3, 256, 1, 64, 3)
     assert fastest({default: 1.0, other: 0.995}) == default
     assert fastest({default: 1.0, other: 0.98}) == other
+    assert fastest({default: 0.104, other: 0.1}) == default and fastest({default: 0.107, other: 0.1}) == other
     assert fastest({other: 1.0, MisLaunch(): 0.999}) == MisLaunch()  # no default among the candidates

@@ -153,30 +153,36 @@ def test_noalloc_under_the_set_default_configuration(gpu):
     bh.free()
 
 
-def test_tuners_keep_the_default_where_it_is_fastest(gpu, tmp_path):
-    """A small frame and a small ray batch: the tuners end on the choice by size (several times faster than any
-    launch that can be set), leave the handle so, and read it back from a cache."""
+def test_tuners_apply_what_they_choose(gpu, tmp_path, monkeypatch):
+    """The tuners leave the handle at the choice by size where they choose the default, read that back from a
+    cache, and set any other choice. (The choice is given: timings are not this test's matter.)"""
     import torch
-    from gonzales_amd.autotune import autotune, autotune_mis
+    from gonzales_amd import autotune as at
 
     integ, cam = _cornell(False)
     n = 30_000
     start = torch.empty(n * abi.GZ_PATH.itemsize, dtype=torch.uint8, device="cuda")
     cam.paths_device(start, 0, n)
-    best, timings = autotune_mis(integ, start, n)
-    assert best.by_size == 1 and integ.launch_by_size(), timings
-    integ.bh.free()
-
-    bh = random_soup_hierarchy(20_000, 3, scale=0.05)
+    bh = random_soup_hierarchy(2000, 3, scale=0.05)
     bh.upload_to_gpu()
-    rays, tmax = random_rays(50_000, 4)
+    rays, tmax = random_rays(5000, 4)
     d = torch.from_numpy(rays.view(np.uint8).reshape(-1)).cuda()
     t = torch.from_numpy(tmax).cuda()
-    best, timings = autotune(bh, d, t, cache=tmp_path / "tuned.json")
-    default = next(c for c in timings if c.by_size)
-    assert timings[best] <= timings[default]
-    assert timings[default] < 0.9 * min(timings[c] for c in timings if c.persistent != 0 and not c.by_size)
+    integ.set_launch(3, 256, 1, 64, 1)
     bh.set_trace_config(3, 8, 32)
-    again, none = autotune(bh, d, t, cache=tmp_path / "tuned.json")
-    assert again == best and none == {} and (bh.trace_config().reserved == abi.GZ_LAUNCH_BY_SIZE) == bool(best.by_size)
+    for k, by_size in ((0, True), (1, False), (0, True)):
+        monkeypatch.setattr(at, "fastest", lambda timings: list(timings)[k])
+        best, timings = at.autotune_mis(integ, start, n, reps=1)
+        assert set(timings) == set(at.MIS_CANDIDATES) and best == at.MIS_CANDIDATES[k]
+        assert integ.launch_by_size() == by_size and (by_size or integ.launch() == (3, 256, 1, 64, 0))
+        cache = tmp_path / f"tuned{k}.json"
+        cache.unlink(missing_ok=True)
+        best, timings = at.autotune(bh, d, t, reps=1, cache=cache)
+        assert set(timings) == set(at.CANDIDATES) and best == at.CANDIDATES[k]
+        assert (bh.trace_config().reserved == abi.GZ_LAUNCH_BY_SIZE) == by_size
+        bh.set_trace_config(1, 8, 32)
+        again, none = at.autotune(bh, d, t, cache=cache)
+        assert again == best and none == {}
+        assert (bh.trace_config().reserved == abi.GZ_LAUNCH_BY_SIZE) == by_size
+    integ.bh.free()
     bh.free()
