@@ -1010,7 +1010,9 @@ static void refresh_default_launch(Scene *s) {
 // 0.85, 3.1M 2.3 and 1.85, so those keep levels, with 128 entries a wave (64: 0.94 and 1.92 ms, 256: 0.85 and
 // 1.92). Scenes whose default is the wavefront, wavefront / whole: 120K paths on a 20K-triangle sphere 2.66 /
 // 1.42, 256K on 200K triangles 3.57 / 1.73, 1M on 300K 5.5 / 4.3 and on a 60K-triangle soup 1.9 / 1.0, 2.9M on
-// 300K 8.3 / 13.7: whole up to 2^20. A trace that keeps a record for the replay runs the levels it records.
+// 300K 8.3 / 13.7: whole up to 2^20, where spheres that fill a square frame cross (300K triangles 0.8M 5.3 /
+// 4.4, 1.05M 6.1 / 6.6; 20K 0.8M 3.9 / 3.5, 1.05M 4.3 / 5.4; 2M 1.05M 8.1 / 8.0). A trace that keeps a record for
+// the replay runs the levels it records.
 struct LaunchChoice {
         GzMisLaunch launch;
         bool wholePaths;

@@ -275,8 +275,9 @@ enum : int { kStepGo = 0, kStepDone = 1, kStepOverflow = 2 };
 // step whatever mix of leaves and interior nodes its lanes stand at. With the triangles loaded inside
 // the leaf branch a wave waited a second time in nearly every other step (a ray tests 1.2 leaves in
 // 125 steps, but 64 lanes do not meet them together), for the whole leaf. 1080p x 8 spp frame of the
-// 327K-triangle displaced sphere: 30.2 -> 25.4 ms; Cornell 512^2 x 16 spp: 3.60 -> 3.01 ms; 100K any-hit
-// rays on 200K triangles: 538 -> 508 us; 16M incoherent rays: 15.4 -> 14.9 ms. Letting lanes wait at a
+// 327K-triangle displaced sphere: 30.7 -> 26.5 ms; Cornell 512^2 x 16 spp: 3.64 -> 3.07 ms; 100K any-hit
+// rays on 200K triangles: 547 -> 518 us; 16M incoherent rays, none with a zero component: 15.36 -> 14.90 ms
+// (each on both sides of this one change). Letting lanes wait at a
 // leaf until 8 or 16 of the wave stand at one was slower (16M rays by 5%, 100K rays by 19% and 35%).
 //
 // `boxes` (Scene::boxes) lets beyond_zero_axis cull; the path kernels pass 0, which takes that code out:

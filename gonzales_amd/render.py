@@ -34,24 +34,28 @@ class FrameRenderer:
     holds about 285 B of device state per path (112 B here, the rest in the scene handle's queue
     storage, one per stream); larger sequences are faster, since every sequence pays each bounce
     level's tail (the chip draining the level's last waves): in one lane the 5M-triangle 1080p x
-    64 spp frame takes 259 ms in 32M-path sequences and 241 ms as one sequence of 132.7M paths
-    (38 GB).
+    64 spp frame took 259 ms in 32M-path sequences and 241 ms as one sequence of 132.7M paths
+    (38 GB; 208 ms with the present kernels).
 
     The frame's pixels are cut into `lanes` contiguous ranges, each rendered on its own stream
     (lane 0 on the caller's stream, the others on streams of the renderer's own that start after
     the work queued on the caller's stream and that the caller's stream waits for at the end), in
     sequences of at most batch_paths / lanes paths with a path buffer per lane: one range's level
-    tails overlap the other's work. The 5M-triangle frame with the same device state: 229-230 ms
-    as two 66M-path lanes against 241 ms as one sequence, 246 ms as two lanes of 16M-path
-    sequences against 259 ms as one lane of 32M-path sequences; the Cornell box at 512^2 x 16 spp
-    (4.2M paths, the queued megakernel) 3.64 against 3.84 ms. lanes = 0 (the default) takes two
-    lanes for frames of at least 4M paths and one below: smaller frames do not fill the chip with
-    one lane's kernels, and their persistent kernels only queue behind each other (the Cornell box
-    at 256^2 x 16 spp: 2.41 ms in two lanes against 1.52 in one). The lanes add to disjoint pixels of the film, and every path's
+    tails overlap the other's work: the 5M-triangle frame 196 ms as two 66M-path lanes against 208
+    ms as one sequence, the Cornell box at 512^2 x 16 spp (4.2M paths, the queued megakernel) 2.75
+    against 2.86 ms. lanes = 0 (the default) takes two lanes for frames of at least 4M paths and one
+    below, where two lanes of up to 2^20 paths each would run their paths whole (the default
+    launch) and lose to one lane's levels. One lane / two in ms: a 300K-triangle sphere 1M paths 6.5 /
+    7.6, 2.1M 7.8 / 11.2, 3.1M 8.9 / 8.3, 4.2M 12.0 / 11.1, 6.3M 12.4 / 11.3, 11.8M 21.5 / 19.6, 16.6M
+    26.7 / 25.0; the Cornell box 1M 0.86 / 0.98, 2.1M 0.96 / 0.90, 3.1M 1.83 / 1.73. Wavefront frames of
+    8.4M paths (two lanes of exactly 2^22) lose, for a reason not found: the sphere 13.4 / 16.9, a
+    300K-triangle soup 8.8 / 12.3.
+    The lanes add to disjoint pixels of the film, and every path's
     result is independent of its sequence, so the film is bit-identical for any lane count and
     batch size. The lanes take equal pixel counts: cutting them so that they end together (by
-    measured lane times) made the 5M-triangle frame slower (235 against 228-230 ms), as the two
-    lanes' level tails then fall together instead of overlapping the other lane's work."""
+    measured lane times) made the 5M-triangle frame slower (235 against 228-230 ms with the kernels of
+    the time), as the two lanes' level tails then fall together instead of overlapping the other
+    lane's work."""
     camera: PerspectiveCamera
     integrator: VolumePathIntegrator
     film: DeviceFilm
